@@ -666,6 +666,13 @@ template <typename T, int AUX> __device__ __forceinline__ cc_v4<T> cc_bld4(__amd
   __builtin_memcpy(&o, &v, 16);
   return o;
 }
+// 16 bytes as the vector V.
+template <typename V> __device__ __forceinline__ V cc_bldv(__amdgpu_buffer_rsrc_t r, int voff) {
+  const cc_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0);
+  V o;
+  __builtin_memcpy(&o, &v, 16);
+  return o;
+}
 template <typename T, int AUX> __device__ __forceinline__ void cc_bst4(__amdgpu_buffer_rsrc_t r, int voff, int soff, const cc_v4<T>& x) {
   static_assert(sizeof(T) == 4, "4-byte elements");
   cc_u32x4 v;
@@ -4650,21 +4657,36 @@ struct Lowering {
   }
 
   // Block tile edge of the matrix-core kernels (square tiles; four waves of
-  // BM/2 x BM/2).
-  static int64_t mfma_bm(DT dt) {
-    if (dt == DT::F64) return tune("mm_f64_bm", 64) == 128 ? 128 : 64;
-    return 128;
+  // BM/2 x BM/2). The large tile reads less per product, but below about
+  // one tile a CU the chip idles and each tile's k loop runs at its memory
+  // latency, so smaller grids take the small tile (and deeper k tiles,
+  // mfma_bk). Measured, large / small tile, us: f32 1024^3 76 / 30,
+  // 1500x2000x1000 (192 large tiles) 84 / 77, 1800x1900x1000 (225) 87 / 92;
+  // f64 512^3 25 / 10, 1000^3 (256) 71 / 56, 1200^3 (361) 81 / 90.
+  static int64_t mfma_bm(DT dt, int64_t M, int64_t N) {
+    if (dt == DT::F64) {
+      const int64_t want = tune("mm_f64_bm", 0);
+      if (want > 0) return want == 128 || want == 32 ? want : 64;
+      return cdiv(M, 64) * cdiv(N, 64) < 300 ? 32 : 64;
+    }
+    return cdiv(M, 128) * cdiv(N, 128) < 208 ? 64 : 128;
   }
-  // k-tile depth: 16, or 32 where K allows it and the knob asks for it.
-  static int64_t mfma_bk(DT dt, int64_t K) {
-    int64_t want = tune(dt == DT::F64 ? "mm_f64_bk" : "mm_bk", 16);
-    return want == 32 && K % 32 == 0 ? 32 : 16;
+  // k-tile depth: 16, deeper for the small tile, whose k loop is short of
+  // work to hide its loads behind (f32 512^3: 22 us at 16, 17 at 32, 15 at
+  // 64; f64 512^3 with the 32-wide tile: 10.5 at 32, 11.0 at 64).
+  static int64_t mfma_bk(DT dt, int64_t M, int64_t N, int64_t K) {
+    const bool small = mfma_bm(dt, M, N) == (dt == DT::F64 ? 32 : 64);
+    int64_t want = tune(dt == DT::F64 ? "mm_f64_bk" : "mm_bk", !small ? 16 : dt == DT::F64 ? 32 : 64);
+    if (K < want) want = K >= 32 ? 32 : 16;
+    return want == 64 || want == 32 ? want : 16;
   }
 
   // ---- Matmul on the matrix cores ------------------------------------------
-  // f32: v_mfma_f32_32x32x2f32, block tile 128x128x16, four waves of 64x64.
-  // f64: v_mfma_f64_16x16x4f64, block tile 64x64x16, four waves of 32x32.
-  // Within a 16-deep k tile, lane group g (of 64/MT groups) takes the k
+  // f32: v_mfma_f32_32x32x2f32, block tile 128x128x16 (64x64x64 for small
+  // grids), four waves of 64x64 (32x32).
+  // f64: v_mfma_f64_16x16x4f64, block tile 64x64x16 (32x32x32), four waves
+  // of 32x32 (16x16).
+  // Within a k tile, lane group g (of 64/MT groups) takes the k
   // values g*S .. g*S+S-1 in order (A and B use the same permutation), so a
   // lane's operands for the whole tile are one contiguous run along k.
   // Each operand is staged in the LDS layout that matches its source:
@@ -4681,7 +4703,13 @@ struct Lowering {
     bool f64 = n.dt == DT::F64;
     std::string T = dt_ctype(n.dt);
     int out = buf_of[t];
-    const int64_t BM = mfma_bm(n.dt), BK = mfma_bk(n.dt, K), MT = f64 ? 16 : 32;
+    const int64_t BM = mfma_bm(n.dt, M, N), BK = mfma_bk(n.dt, M, N, K), MT = f64 ? 16 : 32;
+    // Sides that are no multiple of the tile: operands are read through
+    // buffer resources, whose out-of-range words read zero (rows past the
+    // end of A, k rows past the end of B), and k columns past K are zeroed
+    // in the last k tile. Columns past N read the next row's values; they
+    // reach only outputs that are not stored.
+    const bool ragged = M % BM != 0 || N % BM != 0 || K % BK != 0;
     const int64_t G = 64 / MT;    // lane groups along k
     const int64_t S = BK / G;     // k steps per tile held by one lane
     const int64_t WT = BM / 2;    // wave tile
@@ -4752,16 +4780,34 @@ struct Lowering {
         // thread -> (row r, k offset kk) with PER consecutive k
         l << "    { const int r = threadIdx.x / " << BK / PER << ", kk = (threadIdx.x % " << BK / PER << ") * " << PER
           << ";\n";
+        const std::string mn = mnb + " + r";
         if (o.mode == 2) {
           for (int64_t c = 0; c < PER; c++) {
-            std::string idx = is_a ? "(" + mnb + " + r) * " + std::to_string(K) + " + kt + kk + " + std::to_string(c)
-                                   : "(kt + kk + " + std::to_string(c) + ") * " + std::to_string(N) + " + " + mnb +
-                                         " + r";
-            l << "      " << reg << "[" << c / VEC << "][" << c % VEC << "] = " << o.fn.call_scalar(idx) << ";\n";
+            const std::string kc = "kt + kk + " + std::to_string(c);
+            const std::string idx = is_a ? "(" + mn + ") * " + std::to_string(K) + " + " + kc
+                                         : "(" + kc + ") * " + std::to_string(N) + " + " + mn;
+            l << "      " << reg << "[" << c / VEC << "][" << c % VEC << "] = ";
+            if (ragged)
+              l << "(" << mn << " < " << MNtot << " && " << kc << " < " << K << ") ? " << o.fn.call_scalar(idx) << " : "
+                << zero_of(n.dt) << ";\n";
+            else
+              l << o.fn.call_scalar(idx) << ";\n";
+          }
+        } else if (ragged) {
+          l << "      const int vo = ((" << mn << ") * " << K << " + kt + kk) * " << dt_size(n.dt) << ";\n";
+          for (int64_t c = 0; c < PER; c += VEC)
+            l << "      " << reg << "[" << c / VEC << "] = cc_bldv<" << RV << ">(" << (is_a ? "qa" : "qb") << ", vo + "
+              << c * dt_size(n.dt) << ");\n";
+          if (K % BK != 0) {
+            l << "      if (kt > " << K - BK << ") {\n";
+            for (int64_t c = 0; c < PER; c++)
+              l << "        if (kt + kk + " << c << " >= " << K << ") " << reg << "[" << c / VEC << "][" << c % VEC
+                << "] = " << zero_of(n.dt) << ";\n";
+            l << "      }\n";
           }
         } else {
           // direct A ([M][K]) or transposed B (source [N][K]): row length K
-          l << "      const " << T << "* s = b" << o.buf << " + (size_t)(" << mnb << " + r) * " << K << " + kt + kk;\n";
+          l << "      const " << T << "* s = b" << o.buf << " + (size_t)(" << mn << ") * " << K << " + kt + kk;\n";
           for (int64_t c = 0; c < PER; c += VEC)
             l << "      " << reg << "[" << c / VEC << "] = *(const " << RV << "*)(s + " << c << ");\n";
         }
@@ -4769,11 +4815,18 @@ struct Lowering {
       } else {
         // thread -> (k row kk, MN offset c0) with PER consecutive MN
         l << "    { const int kk = threadIdx.x / " << BM / PER << ", c0 = (threadIdx.x % " << BM / PER << ") * " << PER
-          << ";\n"
-          << "      const " << T << "* s = b" << o.buf << " + (size_t)(kt + kk) * " << MNtot << " + " << mnb
-          << " + c0;\n";
-        for (int64_t c = 0; c < PER; c += VEC)
-          l << "      " << reg << "[" << c / VEC << "] = *(const " << RV << "*)(s + " << c << ");\n";
+          << ";\n";
+        if (ragged) {
+          l << "      const int vo = ((kt + kk) * " << MNtot << " + " << mnb << " + c0) * " << dt_size(n.dt) << ";\n";
+          for (int64_t c = 0; c < PER; c += VEC)
+            l << "      " << reg << "[" << c / VEC << "] = cc_bldv<" << RV << ">(" << (is_a ? "qa" : "qb") << ", vo + "
+              << c * dt_size(n.dt) << ");\n";
+        } else {
+          l << "      const " << T << "* s = b" << o.buf << " + (size_t)(kt + kk) * " << MNtot << " + " << mnb
+            << " + c0;\n";
+          for (int64_t c = 0; c < PER; c += VEC)
+            l << "      " << reg << "[" << c / VEC << "] = *(const " << RV << "*)(s + " << c << ");\n";
+        }
         l << "    }\n";
       }
       return l.str();
@@ -4815,7 +4868,8 @@ struct Lowering {
     std::string accT = f64 ? "cc_f64x4" : "cc_f32x16";
     int64_t NACC = f64 ? 4 : 16;
     std::string mfma = f64 ? "__builtin_amdgcn_mfma_f64_16x16x4f64" : "__builtin_amdgcn_mfma_f32_32x32x2f32";
-    int64_t tiles_m = M / BM, tiles_n = N / BM, ntiles = tiles_m * tiles_n;
+    int64_t tiles_m = cdiv(M, BM), tiles_n = cdiv(N, BM), ntiles = tiles_m * tiles_n;
+    const int64_t nk = cdiv(K, BK);
     // f64: one LDS buffer, refilled between two barriers (the fragments are
     // in registers by the first), and a four-waves-a-SIMD register budget,
     // which also keeps the accumulators in ordinary vector registers: at
@@ -4823,7 +4877,7 @@ struct Lowering {
     // (mm_f64_single=0, mm_f64_waves=0 restore it). f32 measured no gain
     // from either.
     const bool single = f64 && tune("mm_f64_single", 1) != 0;
-    const int64_t waves = f64 ? std::max<int64_t>(0, std::min<int64_t>(8, tune("mm_f64_waves", 4))) : 0;
+    const int64_t waves = f64 && BM == 64 ? std::max<int64_t>(0, std::min<int64_t>(8, tune("mm_f64_waves", 4))) : 0;
     k << "typedef " << T << " " << accT << " __attribute__((ext_vector_type(" << NACC << ")));\n"
       << "extern \"C\" __global__ __launch_bounds__(256) ";
     if (waves > 0) k << "__attribute__((amdgpu_waves_per_eu(" << waves << ", " << waves << "))) ";
@@ -4835,6 +4889,9 @@ struct Lowering {
       // blocks are dispatched round-robin over the 8 XCDs; give each XCD a
       // contiguous run of tiles so its L2 sees shared A row panels.
       << "  int tile = blockIdx.x;\n";
+    if (ntiles % 8 != 0 && ntiles > 8)
+      k << "  { const int x = tile % 8; tile = x * " << ntiles / 8 << " + (x < " << ntiles % 8 << " ? x : " << ntiles % 8
+        << ") + tile / 8; }\n";
     if (ntiles % 8 == 0) {
       const int64_t TX = ntiles / 8, RX = TX % tiles_n == 0 ? TX / tiles_n : 0;
       k << "  tile = (tile % 8) * " << TX << " + tile / 8;\n";
@@ -4845,7 +4902,13 @@ struct Lowering {
         k << "  { const int x = tile / " << TX << ", l = tile - x * " << TX << "; tile = x * " << TX << " + (l % " << RX
           << ") * " << tiles_n << " + l / " << RX << "; }\n";
     }
-    k << "  const int bm = (tile / " << tiles_n << ") * " << BM << ", bn = (tile % " << tiles_n << ") * " << BM << ";\n"
+    k << "  const int bm = (tile / " << tiles_n << ") * " << BM << ", bn = (tile % " << tiles_n << ") * " << BM << ";\n";
+    if (ragged)
+      for (const Opnd *o : {&A, &B})
+        if (o->mode != 2)
+          k << "  const __amdgpu_buffer_rsrc_t " << (o == &A ? "qa" : "qb") << " = cc_rsrc(b" << o->buf << ", "
+            << prog.bufs[o->buf].bytes() << "u);\n";
+    k
       << "  " << accT << " acc[" << RT << "][" << RT << "];\n"
       << "#pragma unroll\n"
       << "  for (int i = 0; i < " << RT << "; i++)\n"
@@ -4859,7 +4922,7 @@ struct Lowering {
     // about 1.7e-4 for one f32 accumulator (and for the interpreter's own
     // sequential sum). KC = mm_chunk_k, 256 by default.
     int64_t KCT = f64 ? 0 : std::max<int64_t>(0, tune("mm_chunk_k", 256) / BK);
-    if (KCT > 0 && (K / BK) % KCT != 0) KCT = 0;
+    if (KCT >= nk) KCT = 0;  // one chunk: nothing to fold
     if (KCT > 0)
       k << "  " << accT << " tot[" << RT << "][" << RT << "];\n"
         << "#pragma unroll\n"
@@ -4869,10 +4932,10 @@ struct Lowering {
     k << "  int kt = 0;\n"
       << gload(A, true, "ra") << gload(B, false, "rb") << lstore(A, "As[0]", "ra") << lstore(B, "Bs[0]", "rb")
       << "  __syncthreads();\n"
-      << "  for (int it = 0; it < " << K / BK << "; it++) {\n"
+      << "  for (int it = 0; it < " << nk << "; it++) {\n"
       << "    const int buf = " << (single ? "0" : "it & 1") << ";\n"
       << "    kt = (it + 1) * " << BK << ";\n"
-      << "    if (it + 1 < " << K / BK << ") {\n"
+      << "    if (it + 1 < " << nk << ") {\n"
       << gload(A, true, "ra") << gload(B, false, "rb") << "    }\n"
       // keeps the scheduler from sinking the next tile's loads to their
       // LDS stores (to save registers), which left them unhidden
@@ -4884,7 +4947,7 @@ struct Lowering {
       << fragload(A, "al", "fa", "wm") << fragload(B, "bl", "fb", "wn");
     if (single)  // every wave holds its fragments: the buffer takes the next tile
       k << "      __syncthreads();\n"
-        << "      if (it + 1 < " << K / BK << ") {\n"
+        << "      if (it + 1 < " << nk << ") {\n"
         << lstore(A, "As[0]", "ra") << lstore(B, "Bs[0]", "rb") << "      }\n";
     k << "#pragma unroll\n"
       << "      for (int s2 = 0; s2 < " << S << "; s2++)\n"
@@ -4895,10 +4958,10 @@ struct Lowering {
       << "(fa[i][s2], fb[j][s2], acc[i][j], 0, 0, 0);\n"
       << "    }\n";
     if (!single)
-      k << "    if (it + 1 < " << K / BK << ") {\n"
+      k << "    if (it + 1 < " << nk << ") {\n"
         << lstore(A, "As[buf ^ 1]", "ra") << lstore(B, "Bs[buf ^ 1]", "rb") << "    }\n";
     if (KCT > 0)
-      k << "    if ((it + 1) % " << KCT << " == 0) {\n"
+      k << "    if ((it + 1) % " << KCT << " == 0" << (nk % KCT != 0 ? " || it + 1 == " + std::to_string(nk) : "") << ") {\n"
         << "#pragma unroll\n"
         << "      for (int i = 0; i < " << RT << "; i++)\n"
         << "#pragma unroll\n"
@@ -4918,7 +4981,9 @@ struct Lowering {
       k << "        const int row = bm + wm + i * 16 + (lane / 16) + 4 * r;\n";
     else
       k << "        const int row = bm + wm + i * 32 + (r / 4) * 8 + (lane / 32) * 4 + (r % 4);\n";
-    k << "        b" << out << "[(size_t)row * " << N << " + col] = " << (KCT > 0 ? "tot" : "acc") << "[i][j][r];\n"
+    k << "        ";
+    if (ragged) k << "if (row < " << M << " && col < " << N << ") ";
+    k << "b" << out << "[(size_t)row * " << N << " + col] = " << (KCT > 0 ? "tot" : "acc") << "[i][j][r];\n"
       << "      }\n"
       << "    }\n"
       << "}\n";
@@ -5020,8 +5085,16 @@ struct Lowering {
     int64_t K = g.ts[n.a].shape[1];
     if (M == 0 || N == 0) return {};
     if (dt_is_float(n.dt) && K > 0 && tune("mm_mfma", 1)) {
-      int64_t BM = mfma_bm(n.dt);
-      if (M % BM == 0 && N % BM == 0 && K % mfma_bk(n.dt, K) == 0) return lower_matmul_mfma(t, M, N, K);
+      const int64_t BM = mfma_bm(n.dt, M, N), z = dt_size(n.dt), most = int64_t(1) << 31;
+      const bool whole = M % BM == 0 && N % BM == 0 && K % mfma_bk(n.dt, M, N, K) == 0;
+      // Byte offsets into the operands, the rows past their ends included,
+      // are 32-bit in the ragged form. Shapes below the lines keep the
+      // 16x16 tiling (f32 130x37x100 and narrower): there a tile is mostly
+      // padding. Against it: f32 1500x700x901 145 -> 33 us, f64 1500x2001x1101
+      // 816 -> 171, f32 65^3 9.0 -> 7.8, f64 100^3 7.6 and 7.6.
+      const bool fits = (M + BM) * K * z < most && (N + BM) * K * z < most && (K + 64) * std::max(M, N) * z < most;
+      if (whole || (fits && std::min(M, N) >= 32 && K >= 48))
+        return lower_matmul_mfma(t, M, N, K);
     }
     ElemFn fa = gen.element_fn("fa_" + id, n.a, false, false);
     ElemFn fb = gen.element_fn("fb_" + id, n.b, false, false);

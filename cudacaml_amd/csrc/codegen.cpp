@@ -649,6 +649,44 @@ template <typename T> __device__ __forceinline__ void cc_st4_nt(T* p, const cc_v
   __builtin_nontemporal_store(v, (v4*)p);
 }
 template <typename T> struct __attribute__((aligned(2 * sizeof(T)))) cc_v2 { T x, y; };
+// 4-wide accesses at any element: the same dwordx4 accesses as cc_v4's,
+// which need no more than 4-byte alignment.
+template <typename T> struct __attribute__((packed, aligned(sizeof(T)))) cc_u4 { T x, y, z, w; };
+template <typename T> __device__ __forceinline__ cc_v4<T> cc_ld4_u(const T* p) {
+  const cc_u4<T> v = *(const cc_u4<T>*)p;
+  return {v.x, v.y, v.z, v.w};
+}
+template <typename T> __device__ __forceinline__ cc_v4<T> cc_ld4_unt(const T* p) {
+  typedef T v4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  const v4 v = __builtin_nontemporal_load((const v4*)p);
+  return {v.x, v.y, v.z, v.w};
+}
+template <typename T> struct __attribute__((packed, aligned(sizeof(T)))) cc_u2 { T x, y; };
+template <typename T> __device__ __forceinline__ cc_v2<T> cc_ld2_u(const T* p) {
+  const cc_u2<T> v = *(const cc_u2<T>*)p;
+  return {v.x, v.y};
+}
+template <typename T> __device__ __forceinline__ cc_v2<T> cc_ld2_unt(const T* p) {
+  typedef T v2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+  const v2 v = __builtin_nontemporal_load((const v2*)p);
+  return {v.x, v.y};
+}
+template <typename T> __device__ __forceinline__ void cc_st2_u(T* p, const cc_v2<T>& r) {
+  *(cc_u2<T>*)p = cc_u2<T>{r.x, r.y};
+}
+template <typename T> __device__ __forceinline__ void cc_st2_unt(T* p, const cc_v2<T>& r) {
+  typedef T v2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+  const v2 v = {r.x, r.y};
+  __builtin_nontemporal_store(v, (v2*)p);
+}
+template <typename T> __device__ __forceinline__ void cc_st4_u(T* p, const cc_v4<T>& r) {
+  *(cc_u4<T>*)p = cc_u4<T>{r.x, r.y, r.z, r.w};
+}
+template <typename T> __device__ __forceinline__ void cc_st4_unt(T* p, const cc_v4<T>& r) {
+  typedef T v4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  const v4 v = {r.x, r.y, r.z, r.w};
+  __builtin_nontemporal_store(v, (v4*)p);
+}
 // Buffer-resource accesses of 16 bytes: a descriptor in scalar registers,
 // one shared per-lane byte offset and a uniform offset, so a run of loads
 // costs one vector register of addressing; out-of-range loads read zero.
@@ -1471,7 +1509,7 @@ struct Lowering {
     const int64_t bytes = root_bytes(r);
     static const char *helpers[] = {"scan_init",          "scatter_zero",   "scatter_count",  "scatter_colscan",
                                     "scatter_bscan",      "scatter_accumulate", "scatter_reduce", "matmul_ksum",
-                                    "reduce_split_fold",  "scatter_coarse",     "gather_slices",  "scatter_windows"};
+                                    "reduce_split_fold",  "scatter_coarse",     "gather_slices",  "scatter_windows", "scan_totals"};
     int main = ks.back();
     for (int k : ks) {
       bool helper = false;
@@ -2395,22 +2433,30 @@ struct Lowering {
   // The tile templates' shape for a row of `len` elements of `dt`: NW waves
   // a workgroup, U slices of SL = 256 NW elements a tile, tiles per row.
   struct TileShape {
-    int64_t NW, U, SL, tile, tpr;
+    int64_t GW, NW, U, SL, tile, tpr;  // GW: elements a thread takes of a slice
   };
   static TileShape tile_shape(int64_t len, DT dt) {
     const bool wide = dt_size(dt) == 8;
-    auto shape = [&](int64_t NW) {
+    auto shape = [&](int64_t NW, int64_t GW) {
       TileShape s;
       s.NW = NW;
-      int64_t Umax = tune(wide ? "lb_slices8" : "lb_slices4", wide ? 8 : (s.NW == 8 ? 13 : 22));
+      s.GW = GW;
+      int64_t Umax = tune(wide ? "lb_slices8" : "lb_slices4", wide ? (GW == 2 ? 12 : 8) : (s.NW == 8 ? 13 : 22));
       if (Umax < 1) throw InvalidArgument("CCHIP_TUNE: look-back slices must be >= 1");
-      s.SL = 256 * s.NW;
+      s.SL = 64 * GW * s.NW;
       s.U = std::min<int64_t>(Umax, std::max<int64_t>(1, cdiv(len, s.SL)));
       s.tile = s.SL * s.U;
       s.tpr = cdiv(len, s.tile);
       return s;
     };
-    return shape(tune("lb_waves", 8) == 8 ? 8 : 4);
+    const int64_t NW = tune("lb_waves", 8) == 8 ? 8 : 4;
+    const TileShape one = shape(NW, 4);
+    // Rows of several tiles take 16 bytes a thread of every slice, so a
+    // wave's access is one contiguous run: 4 elements of 8 bytes would be
+    // two 16-byte accesses 32 bytes apart, each half of every line (2^27
+    // f64: 463 -> 432 us). One-tile rows keep 4, with half the slices to
+    // scan (1500 x 3001 f64: 16.0 us, 17.2 with 2).
+    return wide && one.tpr > 1 ? shape(NW, 2) : one;
   }
 
   // Whether a scan root takes the tile template with one tile a row (one
@@ -2631,9 +2677,9 @@ struct Lowering {
       return {add_kernel(kname, args, grid, 256, "scan_wave")};
     }
     // Rows longer than 64 with few rows: a register-resident tile scan.
-    // A tile is U slices of 1024 elements; thread t holds the 4 contiguous
-    // elements 4t..4t+3 of every slice (one 16-byte load each, all in
-    // flight together). The scan runs in that layout: a 4-element scan per
+    // A tile is U slices of 4 (or 2) elements a thread; thread t holds the
+    // contiguous elements 4t..4t+3 of every slice (one 16-byte load each,
+    // all in flight together). The scan runs in that layout: a 4-element scan per
     // thread, a wave scan of thread totals per slice, one barrier to share
     // the 4 wave totals of every slice, and the slice prefixes are folded
     // in with earlier elements always on the left. When a row spans
@@ -2661,18 +2707,52 @@ struct Lowering {
     // waves stream fastest on gfx950. 4-byte values over 13 slices (26624
     // elements a tile): 2^28 i32 in 381-383 us, against 395-398 us for 4
     // waves over 22 slices, and 386, 396, 392 and 397 us for 8 waves over
-    // 12, 14, 15 and 16 slices. 8-byte values over 8 slices: 2^27 i64 or
-    // f64 in 472-476 us, against 552 us for 4 waves (6 slices: the same;
-    // 4, 5 and 7 slices: 545, 493-519 and 485 us).
-    const TileShape ts = tile_shape(len, n.dt);
+    // 12, 14, 15 and 16 slices. 8-byte values over 12 slices of 1024: 2^27
+    // i64 or f64 in 432 us (14 and 16 slices: 460 and 434, the latter
+    // spilling).
+    TileShape ts = tile_shape(len, n.dt);
+    const int GW = (int)ts.GW;
+    // A whole-tensor scan whose input stays in the 256 MB MALL between two
+    // reads takes two passes instead of the look-back: every tile's total
+    // (scan_totals), then every tile scanned and the totals before it
+    // folded in (scan_carry), in a fixed order. No tile waits for another,
+    // so the tiles can be small (4 slices: more of them in flight, an even
+    // last round); the input's second read is the price. Look-back / two
+    // passes, us: f64 3M 18 / 14.7, 10M 58 / 40, 20M 89 / 88, 40M 151 / 168;
+    // i32 3M 12.5 / 9.0, 10M 21.6 / 21.4, 20M 39.2 / 38.9, 40M 60 / 79.
+    // The input is evaluated twice, so only light functions of it take them
+    // (under 48 lines, as for the folds in maps). scan_carry=0 keeps the
+    // look-back.
+    const bool two_pass = ts.tpr > 1 && rows == 1 && len > (1 << 20) &&
+                          std::max(fn_bytes(f, len), len * dt_size(n.dt)) <= (wide ? int64_t(160) << 20 : int64_t(64) << 20) &&
+                          std::count(f.code.begin(), f.code.end(), '\n') < 48 && any_order(n.body, n.dt, true) && tune("scan_carry", 1) != 0;
+    // Short chains of tiles take fewer slices a tile, for 256 tiles or
+    // more: one CU's load of a large tile is what they wait for (100000
+    // i32: 12.7 us in 26624-element tiles, 7.7 in 4096; 1M f64 14.7 / 12).
+    if (ts.tpr > 1) {
+      const int64_t u = two_pass ? 4 : std::max<int64_t>(2, cdiv(rows * len, ts.SL * 256));
+      if (u < ts.U) {
+        ts.U = u;
+        ts.tile = ts.SL * u;
+        ts.tpr = cdiv(len, ts.tile);
+      }
+    }
     const int64_t NW = ts.NW, SL = ts.SL, NT = 64 * NW, U = ts.U, tile = ts.tile, tpr = ts.tpr;
     int64_t tiles = rows * tpr;
-    bool chained = tpr > 1;
+    bool chained = tpr > 1 && !two_pass;
     if (!reds.empty() && chained) throw Failure("Lower: sibling reductions need one tile a row");
-    bool vec = len % 4 == 0;
+    bool vec = len % GW == 0;
+    // Rows of any other length: the same 4-element groups, read and written
+    // at element alignment. A row's last tile ends inside a group: its
+    // whole groups go as the others do, and the thread that holds the
+    // partial one takes its elements one by one (read from the group that
+    // ends the row where there is none, so no load runs past the row).
+    bool uvec = !vec && len >= GW && dt_size(n.dt) >= 4;
+    for (int b : f.ident) uvec = uvec && dt_size(prog.bufs[b].dt) >= 4;
     int words = wide ? 2 : 1;
     const bool selfsched = chained && !wide && tune("lb_counter", 0) == 0;
     int status = -1, ctr = -1, kinit = -1;
+    if (two_pass) status = add_buf("t" + id + "_totals", n.dt, tpr - 1, BufRole::Scratch);
     if (chained) {
       status = add_buf("t" + id + "_status", DT::I64, tiles * words, BufRole::Scratch);
       if (!selfsched) ctr = add_buf("t" + id + "_tiles", DT::I32, 2, BufRole::Scratch);
@@ -2697,6 +2777,7 @@ struct Lowering {
     p.out.push_back(out);
     for (int o : rout) p.out.push_back(o);
     if (side >= 0) p.out.push_back(side);
+    if (two_pass) p.in.push_back(status);
     if (chained) p.err = true;
     std::vector<int> args;
     std::string params = param_list(p, args);
@@ -2735,7 +2816,7 @@ struct Lowering {
     // whole tile): 4-byte operands under 2 GiB, and an element function
     // without gathers, since lanes past the tile read (and discard) data
     // beyond it.
-    bool bufx = vec && tune("lb_buf", 1) && f.ptrs.empty() && dt_size(n.dt) == 4 &&
+    bool bufx = (vec || uvec) && tune("lb_buf", 1) && f.ptrs.empty() && dt_size(n.dt) == 4 &&
                 prog.bufs[out].bytes() < (int64_t(1) << 31);
     for (int b : f.ident) bufx = bufx && dt_size(prog.bufs[b].dt) == 4 && prog.bufs[b].bytes() < (int64_t(1) << 31);
     // Streaming (non-temporal) accesses, a bit mask: 1 stores, 2 loads.
@@ -2744,17 +2825,108 @@ struct Lowering {
     // 96 -> 89 us: their plain loads leave clean lines in the MALL where
     // streamed ones measured slower; rt_nt=3 streams both).
     int64_t scan_nt = tune(chained ? "scan_nt" : "rt_nt", -1);
+    if (scan_nt < 0 && two_pass) scan_nt = 1;  // the loads are to find the input in the MALL (10M f64 48 -> 40 us)
     if (scan_nt < 0)
-      scan_nt = narrow(f, n.dt) && streams(fn_bytes(f, rows * len) + rows * len * dt_size(n.dt)) ? (chained ? 3 : 1) : 0;
+      scan_nt = (wide || narrow(f, n.dt)) && streams(fn_bytes(f, rows * len) + rows * len * dt_size(n.dt)) ? (chained ? 3 : 1) : 0;
     if (n.dt == DT::BOOL) scan_nt = 0;
     for (int b : f.ident)
       if (prog.bufs[b].dt == DT::BOOL) scan_nt &= ~int64_t(2);
     static const char *comp[] = {"x", "y", "z", "w"};
+    // The tile's elements into v[u][c]: a thread's 4-element group of every
+    // slice, all in flight together.
+    auto load_tile = [&](std::ostringstream &k) {
+      k << "  " << T << " v[" << U << "][" << GW << "];\n"
+        << "#pragma unroll\n"
+        << "  for (int u = 0; u < " << U << "; u++) {\n"
+        << "    const int e = threadIdx.x * " << GW << " + " << SL << " * u;\n";
+      // Groups past the tile read the tile's first group (always valid) and
+      // take init: no load sits behind a branch.
+      if (vec || uvec) {
+        if (uvec)
+          k << "    const bool ok = e + " << GW << " <= tl;\n"
+            << "    const int i = base + (ok ? e : min(0, tl - " << GW << "));\n";
+        else
+          k << "    const bool ok = e < tl;\n"
+            << "    const int i = base + (ok ? e : 0);\n";
+        if (bufx) {
+          for (int b : f.ident)
+            k << "    const cc_v4<" << ty(b) << "> l" << b << " = cc_bld4<" << ty(b) << ", " << ((scan_nt & 2) ? 2 : 0)
+              << ">(r" << b << ", threadIdx.x * 16, (base + " << SL << " * u) * 4);\n";
+        } else if (uvec) {
+          for (int b : f.ident)
+            k << "    const cc_v" << GW << "<" << ty(b) << "> l" << b << " = cc_ld" << GW << "_u" << ((scan_nt & 2) ? "nt" : "")
+              << "(b" << b << " + i);\n";
+        } else {
+          k << vec_loads(f, "i", "    ", tyof(), (scan_nt & 2) != 0, GW);
+        }
+        for (int c = 0; c < GW; c++)
+          k << "    v[u][" << c << "] = ok ? " << lane_call(f, "i", c) << " : " << ini << "();\n";
+      } else {
+        for (int c = 0; c < GW; c++)
+          k << "    { const bool ok = e + " << c << " < tl; const int i = base + (ok ? e + " << c << " : 0); v[u][" << c
+            << "] = ok ? " << f.call_scalar("i") << " : " << ini << "(); }\n";
+      }
+      k << "  }\n";
+      if (uvec) {
+        k << "  if (tl & " << GW - 1 << ") {\n"
+          << "#pragma unroll\n"
+          << "    for (int u = 0; u < " << U << "; u++) {\n"
+          << "      const int e = threadIdx.x * " << GW << " + " << SL << " * u;\n"
+          << "      if (e < tl && e + " << GW << " > tl) {\n";
+        for (int c = 0; c < GW - 1; c++)
+          k << "        if (e + " << c << " < tl) { const int i = base + e + " << c << "; v[u][" << c
+            << "] = " << f.call_scalar("i") << "; }\n";
+        k << "      }\n"
+          << "    }\n"
+          << "  }\n";
+      }
+    };
+    std::string group_scan;
+    for (int c = 1; c < GW; c++)
+      group_scan += strf("    v[u][%d] = %s(v[u][%d], v[u][%d]);\n", c, cmb.c_str(), c - 1, c);
+    auto group_add = [&](const char *x) {
+      std::string r;
+      for (int c = 0; c < GW; c++) r += strf("      v[u][%d] = %s(%s, v[u][%d]);\n", c, cmb.c_str(), x, c);
+      return r;
+    };
     std::ostringstream k;
-    // Four waves per SIMD (at most 128 VGPRs): the fallback's registers
-    // must not cost the main path its occupancy.
+    const std::string S = "b" + std::to_string(status);
+    if (two_pass) {
+      Params pt;
+      add_in(pt, f);
+      pt.out.push_back(status);
+      std::vector<int> targs;
+      const std::string tparams = param_list(pt, targs);
+      std::ostringstream q;
+      q << "extern \"C\" __global__ __launch_bounds__(" << NT << ") void " << kname << "_totals(" << tparams << ") {\n"
+        << "  __shared__ " << T << " wpart[" << NW << "];\n"
+        << "  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;\n"
+        << "  const int base = blockIdx.x * " << tile << ", tl = " << tile << ";\n";
+      if (bufx)
+        for (int b : f.ident)
+          q << "  const __amdgpu_buffer_rsrc_t r" << b << " = cc_rsrc(b" << b << ", " << prog.bufs[b].bytes() << "u);\n";
+      load_tile(q);
+      q << "  " << T << " w = v[0][0];\n"
+        << "#pragma unroll\n"
+        << "  for (int u = 0; u < " << U << "; u++)\n"
+        << "#pragma unroll\n"
+        << "    for (int c = u == 0 ? 1 : 0; c < " << GW << "; c++) w = " << cmb << "(w, v[u][c]);\n";
+      for (int off = 32; off > 0; off /= 2) q << "  w = " << cmb << "(w, __shfl_down(w, " << off << "));\n";
+      q << "  if (lane == 0) wpart[wid] = w;\n"
+        << "  __syncthreads();\n"
+        << "  if (threadIdx.x == 0) {\n"
+        << "    " << T << " t = wpart[0];\n"
+        << "    for (int j = 1; j < " << NW << "; j++) t = " << cmb << "(t, wpart[j]);\n"
+        << "    " << S << "[blockIdx.x] = blockIdx.x == 0 ? " << cmb << "(" << ini << "(), t) : t;\n"
+        << "  }\n"
+        << "}\n";
+      src << q.str();
+      kinit = add_kernel(kname + "_totals", targs, (int)(tpr - 1), (int)NT, "scan_totals");
+    }
+    // Chained tiles: four waves per SIMD (at most 128 VGPRs), so that the
+    // fallback's registers do not cost the main path its occupancy.
     k << "extern \"C\" __global__ __launch_bounds__(" << NT << ") "
-      << (selfsched ? "__attribute__((amdgpu_waves_per_eu(4))) " : "") << "void " << kname << "(" << params;
+      << (chained ? "__attribute__((amdgpu_waves_per_eu(4))) " : "") << "void " << kname << "(" << params;
     if (chained) k << ", cc_u64* __restrict__ st" << (selfsched ? "" : ", int* __restrict__ ctr");
     k << ") {\n"
       << "  __shared__ " << T << " wsum[" << U << "][" << NW << "];\n"
@@ -2780,30 +2952,28 @@ struct Lowering {
         k << "  const __amdgpu_buffer_rsrc_t r" << b << " = cc_rsrc(b" << b << ", " << prog.bufs[b].bytes() << "u);\n";
       k << "  const __amdgpu_buffer_rsrc_t ro = cc_rsrc(b" << out << ", " << prog.bufs[out].bytes() << "u);\n";
     }
-    k << "  " << T << " v[" << U << "][4];\n"
-      << "#pragma unroll\n"
-      << "  for (int u = 0; u < " << U << "; u++) {\n"
-      << "    const int e = threadIdx.x * 4 + " << SL << " * u;\n";
-    // Groups past the tile read the tile's first group (always valid) and
-    // take init: no load sits behind a branch.
-    if (vec) {
-      k << "    const bool ok = e < tl;\n"
-        << "    const int i = base + (ok ? e : 0);\n";
-      if (bufx) {
-        for (int b : f.ident)
-          k << "    const cc_v4<" << ty(b) << "> l" << b << " = cc_bld4<" << ty(b) << ", " << ((scan_nt & 2) ? 2 : 0)
-            << ">(r" << b << ", threadIdx.x * 16, (base + " << SL << " * u) * 4);\n";
-      } else {
-        k << vec_loads(f, "i", "    ", tyof(), (scan_nt & 2) != 0);
-      }
-      for (int c = 0; c < 4; c++)
-        k << "    v[u][" << c << "] = ok ? " << lane_call(f, "i", c) << " : " << ini << "();\n";
-    } else {
-      for (int c = 0; c < 4; c++)
-        k << "    { const bool ok = e + " << c << " < tl; const int i = base + (ok ? e + " << c << " : 0); v[u][" << c
-          << "] = ok ? " << f.call_scalar("i") << " : " << ini << "(); }\n";
+    const int64_t PC = two_pass ? cdiv(tpr - 1, NT) : 0;  // earlier tiles' totals a thread
+    if (two_pass) {
+      k << "  __shared__ " << T << " wpfx[" << NW << "];\n"
+        << "  " << T << " pt[" << PC << "];\n"
+        << "#pragma unroll\n"
+        << "  for (int c = 0; c < " << PC << "; c++) pt[c] = " << S << "[min((int)threadIdx.x * " << PC << " + c, "
+        << tpr - 2 << ")];\n";
     }
-    k << "  }\n";
+    load_tile(k);
+    if (two_pass) {
+      k << "  {\n"
+        << "    const int active = (tin + " << PC - 1 << ") / " << PC << " - 64 * wid;\n"
+        << "    " << T << " w = pt[0];\n"
+        << "#pragma unroll\n"
+        << "    for (int c = 1; c < " << PC << "; c++) { const " << T << " x = " << cmb
+        << "(w, pt[c]); w = (int)threadIdx.x * " << PC << " + c < tin ? x : w; }\n";
+      for (int off = 1; off < 64; off *= 2)
+        k << "    { const " << T << " o = " << cmb << "(w, __shfl_down(w, " << off << ")); w = lane + " << off
+          << " < active ? o : w; }\n";
+      k << "    if (lane == 0) wpfx[wid] = w;\n"
+        << "  }\n";
+    }
     // Sibling reductions: each lane folds its elements in row order (slice
     // by slice) before the scan changes them, then the wave in a butterfly;
     // one partial a wave goes to LDS with the scan's wave totals.
@@ -2813,9 +2983,9 @@ struct Lowering {
         << "  bool " << Hs << " = false;\n"
         << "#pragma unroll\n"
         << "  for (int u = 0; u < " << U << "; u++) {\n"
-        << "    const int e = threadIdx.x * 4 + " << SL << " * u;\n"
+        << "    const int e = threadIdx.x * " << GW << " + " << SL << " * u;\n"
         << "#pragma unroll\n"
-        << "    for (int c = 0; c < 4; c++) {\n"
+        << "    for (int c = 0; c < " << GW << "; c++) {\n"
         << "      const bool ok_ = e + c < tl;\n"
         << "      const " << rT[j] << " y_ = " << Hs << " ? " << rcmb[j] << "(" << A << ", v[u][c]) : v[u][c];\n"
         << "      " << A << " = ok_ ? y_ : " << A << "; " << Hs << " = " << Hs << " || ok_;\n"
@@ -2829,17 +2999,13 @@ struct Lowering {
     k << "  if (tin == 0 && threadIdx.x == 0) v[0][0] = " << cmb << "(" << ini << "(), v[0][0]);\n"
       << "#pragma unroll\n"
       << "  for (int u = 0; u < " << U << "; u++) {\n"
-      << "    v[u][1] = " << cmb << "(v[u][0], v[u][1]);\n"
-      << "    v[u][2] = " << cmb << "(v[u][1], v[u][2]);\n"
-      << "    v[u][3] = " << cmb << "(v[u][2], v[u][3]);\n"
-      << "    " << T << " incl = v[u][3];\n";
+      << group_scan << "    " << T << " incl = v[u][" << GW - 1 << "];\n";
     for (int off = 1; off < 64; off *= 2)
       k << "    { const " << T << " o = __shfl_up(incl, " << off << "); if (lane >= " << off << ") incl = " << cmb
         << "(o, incl); }\n";
     // the wave's exclusive prefix is folded in at once (no register per slice kept for it)
     k << "    { const " << T << " ex = __shfl_up(incl, 1);\n"
-      << "      if (lane > 0) { v[u][0] = " << cmb << "(ex, v[u][0]); v[u][1] = " << cmb << "(ex, v[u][1]);\n"
-      << "                      v[u][2] = " << cmb << "(ex, v[u][2]); v[u][3] = " << cmb << "(ex, v[u][3]); } }\n"
+      << "      if (lane > 0) {\n" << group_add("ex") << "      } }\n"
       << "    if (lane == 63) wsum[u][wid] = incl;\n"
       << "  }\n"
       << "  __syncthreads();\n"
@@ -2850,8 +3016,7 @@ struct Lowering {
       << "    " << T << " pf = run;\n"
       << "    for (int w = 0; w < wid; w++) { pf = hp ? " << cmb << "(pf, wsum[u][w]) : wsum[u][w]; hp = true; }\n"
       << "    if (hp) {\n"
-      << "      v[u][0] = " << cmb << "(pf, v[u][0]); v[u][1] = " << cmb << "(pf, v[u][1]);\n"
-      << "      v[u][2] = " << cmb << "(pf, v[u][2]); v[u][3] = " << cmb << "(pf, v[u][3]);\n"
+      << group_add("pf")
       << "    }\n"
       << "    " << T << " su = wsum[u][0];\n"
       << "#pragma unroll\n"
@@ -3007,41 +3172,59 @@ struct Lowering {
         << "    const " << T << " pfx = s_prefix;\n"
         << "#pragma unroll\n"
         << "    for (int u = 0; u < " << U << "; u++) {\n"
-        << "      v[u][0] = " << cmb << "(pfx, v[u][0]); v[u][1] = " << cmb << "(pfx, v[u][1]);\n"
-        << "      v[u][2] = " << cmb << "(pfx, v[u][2]); v[u][3] = " << cmb << "(pfx, v[u][3]);\n"
+        << group_add("pfx")
         << "    }\n"
         << "  }\n";
     }
+    if (two_pass)
+      k << "  if (tin > 0) {\n"
+        << "    const int nw = (tin + " << 64 * PC - 1 << ") / " << 64 * PC << ";\n"
+        << "    " << T << " pfx = wpfx[0];\n"
+        << "    for (int w = 1; w < nw; w++) pfx = " << cmb << "(pfx, wpfx[w]);\n"
+        << "#pragma unroll\n"
+        << "    for (int u = 0; u < " << U << "; u++) {\n"
+        << group_add("pfx")
+        << "    }\n"
+        << "  }\n";
     k << "#pragma unroll\n"
       << "  for (int u = 0; u < " << U << "; u++) {\n"
-      << "    const int e = threadIdx.x * 4 + " << SL << " * u;\n";
-    if (vec) {
-      k << "    if (e < tl) {\n"
-        << "      cc_v4<" << T << "> o;\n";
-      for (int c = 0; c < 4; c++) k << "      o." << comp[c] << " = v[u][" << c << "];\n";
+      << "    const int e = threadIdx.x * " << GW << " + " << SL << " * u;\n";
+    if (vec || uvec) {
+      k << "    if (e" << (uvec ? " + " + std::to_string(GW) + " <=" : " <") << " tl) {\n"
+        << "      cc_v" << GW << "<" << T << "> o;\n";
+      for (int c = 0; c < GW; c++) k << "      o." << comp[c] << " = v[u][" << c << "];\n";
       if (bufx)
         k << "      cc_bst4<" << T << ", " << ((scan_nt & 1) ? 2 : 0)
           << ">(ro, threadIdx.x * 16, (base + " << SL << " * u) * 4, o);\n";
+      else if (uvec)
+        k << "      cc_st" << GW << "_u" << ((scan_nt & 1) ? "nt" : "") << "(b" << out << " + base + e, o);\n";
       else if (scan_nt & 1)
-        k << "      cc_st4_nt(b" << out << " + base + e, o);\n";
+        k << "      cc_st" << GW << "_nt(b" << out << " + base + e, o);\n";
       else
-        k << "      *(cc_v4<" << T << ">*)(b" << out << " + base + e) = o;\n";
-      k << "    }\n";
+        k << "      *(cc_v" << GW << "<" << T << ">*)(b" << out << " + base + e) = o;\n";
+      k << "    }";
+      if (uvec) {
+        k << " else if (e < tl) {\n";
+        for (int c = 0; c < GW - 1; c++)
+          k << "      if (e + " << c << " < tl) b" << out << "[base + e + " << c << "] = v[u][" << c << "];\n";
+        k << "    }";
+      }
+      k << "\n";
     } else {
-      for (int c = 0; c < 4; c++)
+      for (int c = 0; c < GW; c++)
         k << "    if (e + " << c << " < tl) b" << out << "[base + e + " << c << "] = v[u][" << c << "];\n";
     }
     // the row's last element, held by one thread of the row's last tile
     if (side >= 0)
       k << "    if (tin == " << tpr - 1 << ")\n"
         << "#pragma unroll\n"
-        << "      for (int c = 0; c < 4; c++) if (e + c == tl - 1) b" << side << "[row] = v[u][c];\n";
+        << "      for (int c = 0; c < " << GW << "; c++) if (e + c == tl - 1) b" << side << "[row] = v[u][c];\n";
     k << "  }\n"
       << "}\n";
     src << k.str();
     int kscan = add_kernel(kname, args, (int)tiles, (int)NT,
-                           chained ? "scan_lookback" : reds.empty() ? "scan_tile" : "scan_tile_fold");
-    if (chained) return {kinit, kscan};
+                           chained ? "scan_lookback" : two_pass ? "scan_carry" : reds.empty() ? "scan_tile" : "scan_tile_fold");
+    if (chained || two_pass) return {kinit, kscan};
     return {kscan};
   }
 

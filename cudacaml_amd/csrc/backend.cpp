@@ -94,7 +94,7 @@ struct cchip_program {
   // total, which outputs are copied rather than written in place, and host
   // arrays sized here so that such a run allocates no memory at all.
   std::vector<int64_t> na_off;
-  int64_t na_bytes = 0;
+  int64_t na_bytes = 0, na_counted = 0;
   std::vector<char> na_out_copy;
   std::vector<int> na_which;
   std::vector<void *> na_ptr, na_vals, na_args;
@@ -436,13 +436,18 @@ void prepare_noalloc(cchip_program *p) {
   const ProgramIR &ir = p->ir;
   p->na_off.assign(ir.bufs.size(), -1);
   if (ir.err_buf >= 0) p->na_off[ir.err_buf] = 0;
-  int64_t at = 256;
+  int64_t at = 256, small = 0;
   for (size_t b = 0; b < ir.bufs.size(); b++)
     if (ir.bufs[b].role == BufRole::Scratch) {
       p->na_off[b] = at;
-      at += (std::max<int64_t>(ir.bufs[b].bytes(), 1) + 255) & ~int64_t(255);
+      const int64_t room = (std::max<int64_t>(ir.bufs[b].bytes(), 1) + 255) & ~int64_t(255);
+      at += room;
+      if (room <= (256 << 10)) small += room;
     }
   p->na_bytes = at;
+  // tile words and totals of scans and the like, up to 1 MiB of them, have
+  // room of their own beside the 32 MiB
+  p->na_counted = at - std::min<int64_t>(small, noalloc_scratch_spare());
   p->na_out_copy.assign(ir.outputs.size(), 0);
   std::vector<char> bound(ir.bufs.size(), 0);
   for (auto &ps : ir.params) bound[ps.buf] = 1;
@@ -719,7 +724,7 @@ int cchip_program_run_resident_noalloc(cchip_program *p, int n, const char *cons
     if (p->released) throw Failure("Executor.run_resident: this executor has been released");
     const ProgramIR &ir = p->ir;
     const size_t cap = noalloc_scratch_capacity();
-    if (p->na_bytes > (int64_t)cap)
+    if (p->na_counted > (int64_t)cap)
       throw InvalidArgument(strf("run_resident_noalloc: program %s needs %lld bytes of scratch, more than the "
                                  "%zu bytes of the static scratch",
                                  ir.name.c_str(), (long long)p->na_bytes, cap));

@@ -3334,6 +3334,15 @@ struct Lowering {
     return l.str();
   }
 
+  // Workgroups a slice and partition tile of the scatter being lowered.
+  int64_t sc_wgs = 1, sc_tile = 8192;
+  // Scratch bytes of a tile-local partition and its accumulate.
+  static int64_t local_scratch(int64_t N, int64_t P, int64_t S, int64_t W, int64_t tile, int64_t ES, bool back) {
+    const int64_t G = std::max<int64_t>(1, std::min<int64_t>(std::max<int64_t>(1024, cdiv(N, tile)), cdiv(N, 4096)));
+    const int64_t C = cdiv(cdiv(N, G), 256) * 256, ntt = cdiv(N, C) * cdiv(C, tile), rs = std::min(tile, C) + 8 * P;
+    return ntt * (rs * (2 + ES) + 8 * (P + 1)) + (back ? 2 * N : 0) + (W > 1 ? W * P * S * ES : 0);
+  }
+
   std::vector<int> lower_scatter_lds(int t, int64_t B, int64_t N, int64_t S, int64_t P) {
     const TNode &n = g.ts[t];
     std::string id = std::to_string(n.id);
@@ -3417,8 +3426,9 @@ struct Lowering {
     // Workgroups per slice, about 512 in all: for 2^26 values into 2^20
     // bins (64 slices of 16384, 8 each) the accumulate takes 121 us and the
     // fixed-order sum of the partial tables 11 us, against 132 and 17 us
-    // with 16 each.
-    int64_t W = std::max<int64_t>(1, std::min<int64_t>(16, tune("scatter_slice_wgs", 512) / P));
+    // with 16 each. No fewer than 8192 values each, so that a small input
+    // does not sum more partial table than it has values.
+    int64_t W = sc_wgs;
     while (W > 1 && W * P * S * ES > (int64_t(256) << 20)) W--;
     int part = finish(W, P, P * S);
     std::string sB = std::to_string(B);
@@ -3426,7 +3436,10 @@ struct Lowering {
     // buckets (runs twice as long per bucket as with 4096, at half the
     // occupancy: config 3's partition 323 -> 278 us, config 3b's coarse
     // pass 302 -> 269 us), 4096 above (config 3b's fine pass: 339 against
-    // 409 us); scatter_tile forces one size.
+    // 409 us), for 8-byte values (20M f64 into 100000: 340 -> 308 us a
+    // step) and for inputs of up to 2^23, of which tiles of 8192 are a
+    // round and a bit of workgroups (5M i32 into 10^6: 117 -> 93 us);
+    // scatter_tile forces one size.
     // 1024 threads per staged partition workgroup (config 3's partition
     // 320 -> 288 us, config 3b's passes 313 / 370 -> 282 / 295 us, against
     // 256; 512 is in between); 256 and 512 by scatter_part_threads.
@@ -3435,7 +3448,7 @@ struct Lowering {
     auto tile_of = [&](int64_t PB) -> int64_t {
       const int64_t t = tune("scatter_tile", 0);
       if (t == 4096 || t == 8192) return t;
-      return PB <= 1024 ? 8192 : 4096;
+      return PB <= 1024 ? sc_tile : 4096;
     };
 
     // One partition pass: elements [0, nvalid) of an input stream are
@@ -4133,9 +4146,11 @@ struct Lowering {
       // more threads keep more loads in flight. 1024 where a slice has
       // several workgroups (config 3: 0.545 ms a step against 0.552 with
       // 512), 512 where it has one, whose workgroups are short (config 3b:
-      // 1.071 against 1.104 ms); scatter_acc_threads=256, 512 or 1024
+      // 1.071 against 1.104 ms), or where the table is at most 32 KiB and
+      // leaves room for more of them (5M i32 into 100003 bins, 16 KiB
+      // tables: 93 -> 65 us a step); scatter_acc_threads=256, 512 or 1024
       // forces one.
-      const int64_t at_default = W == 1 ? 512 : 1024;
+      const int64_t at_default = W == 1 || S * ES <= 32768 ? 512 : 1024;
       const int64_t AT = tune("scatter_acc_threads", at_default) == 256    ? 256
                          : tune("scatter_acc_threads", at_default) == 512  ? 512
                          : tune("scatter_acc_threads", at_default) == 1024 ? 1024
@@ -4283,22 +4298,58 @@ struct Lowering {
     return ks;
   }
 
-  // out[b] = sum over w of part[w * stride + b], w ascending.
+  // out[b] = sum over w of part[w * stride + b]. A wave takes 64 bins and
+  // an equal share of the partials, eight loads in flight, w ascending; the
+  // waves' sums are added in order. One wave's share is at most 16 partials
+  // where 16 waves allow it: a thread a bin over all of them left a few
+  // workgroups waiting out one load after another (611 partials of 3000
+  // bins: 41 us).
   int scatter_reduce(const std::string &kname, const std::string &T, const std::string &acc, int part, int out,
                      int64_t W, int64_t B, int64_t stride) {
+    int64_t G = 1;
+    while (G < 16 && W > 16 * G) G *= 2;
+    const int64_t C = cdiv(W, G);
     std::ostringstream k;
-    k << "extern \"C\" __global__ __launch_bounds__(256) void " << kname << "_reduce(const " << T
-      << "* __restrict__ b" << part << ", " << T << "* __restrict__ b" << out << ") {\n"
-      << "  for (int b = blockIdx.x * 256 + threadIdx.x; b < " << B << "; b += gridDim.x * 256) {\n"
-      << "    " << acc << " s = (" << acc << ")b" << part << "[b];\n"
-      << "    for (int w = 1; w < " << W << "; w++) s += (" << acc << ")b" << part << "[(size_t)w * " << stride
-      << " + b];\n"
+    const std::string P = "b" + std::to_string(part);
+    if (G == 1) {
+      k << "extern \"C\" __global__ __launch_bounds__(256) void " << kname << "_reduce(const " << T << "* __restrict__ "
+        << P << ", " << T << "* __restrict__ b" << out << ") {\n"
+        << "  const int b = blockIdx.x * 256 + threadIdx.x;\n"
+        << "  if (b >= " << B << ") return;\n"
+        << "  " << acc << " x[" << W << "];\n"
+        << "#pragma unroll\n"
+        << "  for (int w = 0; w < " << W << "; w++) x[w] = (" << acc << ")" << P << "[(size_t)w * " << stride << " + b];\n"
+        << "#pragma unroll\n"
+        << "  for (int w = 1; w < " << W << "; w++) x[0] += x[w];\n"
+        << "  b" << out << "[b] = (" << T << ")x[0];\n"
+        << "}\n";
+      src << k.str();
+      return add_kernel(kname + "_reduce", {part, out}, (int)cdiv(B, 256), 256, "scatter_reduce");
+    }
+    k << "extern \"C\" __global__ __launch_bounds__(" << 64 * G << ") void " << kname << "_reduce(const " << T
+      << "* __restrict__ " << P << ", " << T << "* __restrict__ b" << out << ") {\n"
+      << "  __shared__ " << acc << " sums[" << G << "][64];\n"
+      << "  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;\n"
+      << "  const int b = blockIdx.x * 64 + lane, bc = min(b, " << B - 1 << ");\n"
+      << "  const int hi = min(" << W << ", (wid + 1) * " << C << ");\n"
+      << "  " << acc << " s = (" << acc << ")0;\n"
+      << "  for (int w0 = wid * " << C << "; w0 < hi; w0 += 8) {\n"
+      << "    " << acc << " x[8];\n"
+      << "#pragma unroll\n"
+      << "    for (int u = 0; u < 8; u++) x[u] = (" << acc << ")" << P << "[(size_t)min(w0 + u, " << W - 1 << ") * " << stride
+      << " + bc];\n"
+      << "#pragma unroll\n"
+      << "    for (int u = 0; u < 8; u++) s += w0 + u < hi ? x[u] : (" << acc << ")0;\n"
+      << "  }\n"
+      << "  sums[wid][lane] = s;\n"
+      << "  __syncthreads();\n"
+      << "  if (wid == 0 && b < " << B << ") {\n"
+      << "    for (int w = 1; w < " << G << "; w++) s += sums[w][lane];\n"
       << "    b" << out << "[b] = (" << T << ")s;\n"
       << "  }\n"
       << "}\n";
     src << k.str();
-    return add_kernel(kname + "_reduce", {part, out}, (int)std::min<int64_t>(cdiv(B, 256), 4096), 256,
-                      "scatter_reduce");
+    return add_kernel(kname + "_reduce", {part, out}, (int)cdiv(B, 64), (int)(64 * G), "scatter_reduce");
   }
 
   // An i32 tensor that is exactly a*i + b in its flat element index i:
@@ -4375,13 +4426,37 @@ struct Lowering {
       // Slices of 16384 bins where the table fits 64 KiB of LDS (8192 for
       // 8-byte types): the longer a slice, the longer each tile's run of it
       // (config 3, 2^20 bins: 640 -> 614 us against 8192). A table of 128
-      // KiB a workgroup (scatter_slice_lds=131072) is allowed too.
+      // KiB a workgroup (scatter_slice_lds=131072) is allowed too. Smaller
+      // tables that need several slices take shorter ones, down to 4096
+      // bins, while they are at most 64: few slices leave most CUs without
+      // a workgroup in the accumulate and put each bin's collisions on few
+      // LDS tables (5M i32 into 20000 bins, 2 slices -> 5: 155 -> 82 us a
+      // step, 20M into 100000, 7 -> 25: 218 -> 179).
       const int64_t lds = tune("scatter_slice_lds", 65536) == 131072 ? 131072 : 65536;
+      const int64_t want = tune("scatter_slice_bins", 0);
+      int64_t top = 4096;
+      while (top < (want > 0 ? want : 16384) && top * 2 * ES <= lds) top *= 2;
+      while (cdiv(M, top) > 4096 && top * ES < lds) top *= 2;
       int64_t S = 4096;
-      const int64_t want = tune("scatter_slice_bins", 16384);
-      while (S < want && S * 2 * ES <= lds) S *= 2;
-      while (cdiv(M, S) > 4096 && S * ES < lds) S *= 2;
+      while (S < top && (want > 0 || M <= top || cdiv(M, S) > 64)) S *= 2;
       int64_t P = cdiv(M, S);
+      sc_wgs = std::max<int64_t>(1, std::min<int64_t>(64, tune("scatter_slice_wgs", 512) / P));
+      sc_wgs = std::min<int64_t>(sc_wgs, std::max<int64_t>(2, N / (P * 8192)));
+      sc_tile = P <= tune("scatter_local_max", 256) && (ES == 8 || N <= (8 << 20)) ? 4096 : 8192;
+      // Shorter slices and tiles may not cost scratch: no more than slices
+      // of `top` bins, tiles of 8192 and up to 16 workgroups a slice take
+      // (runs that fit the static scratch keep fitting it).
+      if (want == 0 && P > 1 && P <= 256) {
+        const int64_t P0 = cdiv(M, top), W0 = std::max<int64_t>(1, std::min<int64_t>(16, tune("scatter_slice_wgs", 512) / P0));
+        bool back0 = false;
+        for (int r : plan.roots) back0 |= g.ts[r].kind == TK::Gather && g.ts[r].b == t && g.ts[r].a == n.a;
+        const int64_t most = local_scratch(N, P0, top, W0, 8192, ES, back0);
+        const bool back = gbp_root_of.count(t) > 0;
+        auto over = [&] { return local_scratch(N, P, S, sc_wgs, sc_tile, ES, back) > most; };
+        while (over() && sc_wgs > 1) sc_wgs--;
+        if (over()) sc_tile = 8192;
+        if (over()) S = top, P = P0, sc_wgs = W0;
+      }
       // Two levels with the slice pass in windows take up to 8192 slices
       // (128 super-slices); the counted forms up to 4096.
       const bool windows = P > tune("scatter_stage_p", 512) && tune("scatter_two_level", 1) && tune("scatter_windows", 1);
@@ -5564,6 +5639,20 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     return {add_kernel(kname, args, (int)cdiv(N, 16), 256, "matmul_tiled", (int)cdiv(M, 16))};
   }
 
+  // Whether a gather of scatter `S`'s table over its own index is faster
+  // read plainly than back through the partition. A plain read is one L2
+  // request an element, at a rate that does not depend on its width while
+  // the table stays in an XCD's 4 MiB L2; the way back moves the values
+  // twice more. Back / plain, us a step: f64 5M into 100003 110 / 85, 20M
+  // into 100000 308 / 244, 20M into 10^6 (8 MB) 367 / 377, 2^19 much the
+  // same either way; i32 5M into 20000 75 / 54, 5M into 100003 65 / 63, 20M
+  // into 100000 161 / 178.
+  bool plain_gather(int S) const {
+    const int64_t N = g.ts[g.ts[S].a].numel, table = g.ts[S].numel * dt_size(g.ts[S].dt);
+    if (dt_size(g.ts[S].dt) == 8) return N > (2 << 20) && table <= (4 << 20);
+    return N > (2 << 20) && N <= (8 << 20) && table <= (256 << 10);
+  }
+
   // Uniform roots (broadcasts, and maps of them that do not use the
   // element index) whose buffer no other root's kernel reads (their
   // consumers compute the value instead; see Gen::elem) and that the graph
@@ -5624,7 +5713,7 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
         const TNode &n = g.ts[r];
         if (n.kind != TK::Gather) continue;
         const int S = n.b;
-        if (g.ts[S].kind == TK::Scatter && g.ts[S].a == n.a && !gbp_root_of.count(S)) gbp_root_of[S] = r;
+        if (g.ts[S].kind == TK::Scatter && g.ts[S].a == n.a && !gbp_root_of.count(S) && !plain_gather(S)) gbp_root_of[S] = r;
       }
     // Scatters with an injective affine index in range are computed where
     // they are read (Gen::scatter_inline_; scatter_inline=0 reads their

@@ -202,6 +202,7 @@ std::vector<char> jit_code_object(const std::string &name, const std::string &so
 
 // The static scratch of the allocation-free entry point (noalloc.hip).
 size_t noalloc_scratch_capacity();
+size_t noalloc_scratch_spare();
 void *noalloc_scratch(int device);
 void noalloc_scratch_clear(void *base, size_t bytes, void *stream);
 

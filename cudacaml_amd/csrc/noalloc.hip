@@ -18,12 +18,13 @@
 
 namespace {
 constexpr size_t kScratchBytes = size_t(32) << 20;
+constexpr size_t kSpareBytes = size_t(1) << 20;  // for buffers of at most 256 KiB, not counted against the 32 MiB
 }
 
 // In host code this name is a host-side stand-in for the device array, not
 // a device address: only the pointer hipGetSymbolAddress returns for the
 // current device may be passed to kernels or copies.
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kSpareBytes];
 
 namespace {
 
@@ -43,6 +44,7 @@ void *g_base[kMaxDevices];
 namespace cchip {
 
 size_t noalloc_scratch_capacity() { return kScratchBytes; }
+size_t noalloc_scratch_spare() { return kSpareBytes; }
 
 // The array's device address on `device`, looked up once per device with
 // that device current (the caller makes it current).

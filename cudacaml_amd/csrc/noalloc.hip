@@ -66,7 +66,7 @@ void *noalloc_scratch(int device) {
 // Queues a zero fill of the first `bytes` of the scratch at `base` (an
 // address noalloc_scratch returned) on `stream`.
 void noalloc_scratch_clear(void *base, size_t bytes, void *stream) {
-  if (bytes > kScratchBytes) throw InvalidArgument("noalloc scratch: clear beyond the array");
+  if (bytes > kScratchBytes + kSpareBytes) throw InvalidArgument("noalloc scratch: clear beyond the array");
   size_t n16 = (bytes + 15) / 16;
   if (!n16) return;
   unsigned grid = (unsigned)std::min<size_t>((n16 + 255) / 256, 1024);

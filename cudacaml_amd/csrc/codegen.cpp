@@ -2084,6 +2084,82 @@ struct Lowering {
     return x.op == B_ADD || x.op == B_MUL || x.op == B_AND || x.op == B_OR || x.op == B_XOR;
   }
 
+  // One-element maps computed by the kernel that ends a reduction to one
+  // value: reduce root -> map roots, in plan order. A kernel of one thread
+  // costs its launch and its cold instruction, argument and operand reads
+  // (4.8 us each beside 2^24-element maps, 1.4 alone); the thread that has
+  // the total computes them from its register. A map joins when everything
+  // else it reads is ready before the reduction (parameters and earlier
+  // roots) and it reads the total by value (scalar_tail=0: its own kernel).
+  std::map<int, std::vector<int>> tails;
+  std::set<int> tail_member;
+  void find_tails() {
+    if (!tune("scalar_tail", 1)) return;
+    std::map<int, size_t> ready;  // buffer -> place of the root that writes it
+    for (size_t i = 0; i < plan.roots.size(); i++) ready[buf_of[plan.roots[i]]] = i;
+    for (size_t ri = 0; ri < plan.roots.size(); ri++) {
+      const int r = plan.roots[ri];
+      const TNode &n = g.ts[r];
+      if (n.kind != TK::Reduce || n.numel != 1 || n.dt == DT::BOOL || sib_member.count(r) || sib_lead.count(r)) continue;
+      if (!fused_part_of(r) && row_length(g.ts[n.a].shape) <= 2048) continue;
+      std::set<int> mine = {buf_of[r]};
+      for (size_t ti = ri + 1; ti < plan.roots.size(); ti++) {
+        const int t = plan.roots[ti];
+        const TNode &m = g.ts[t];
+        if ((m.kind != TK::Map && m.kind != TK::Map2 && m.kind != TK::Reshape) || m.numel != 1 || m.dt == DT::BOOL || gen.uniform(t) ||
+            tail_member.count(t) || fused_red_of_map.count(t) || gen.rowlast_.count(t))
+          continue;
+        const ElemFn f = gen.element_fn("fz_", t, true, true);
+        bool ok = !f.uses_err, reads = false;
+        for (int b : f.ptrs) ok = ok && !mine.count(b) && early(b, ri, ready);
+        for (int b : f.ident) {
+          reads = reads || mine.count(b);
+          ok = ok && (mine.count(b) || early(b, ri, ready));
+        }
+        if (!ok || !reads) continue;
+        tails[r].push_back(t);
+        tail_member.insert(t);
+        mine.insert(buf_of[t]);
+      }
+    }
+  }
+  bool fused_part_of(int r) const {
+    for (auto &fr : fused_red_of_map)
+      if (fr.second == r) return true;
+    return false;
+  }
+  // Whether buffer b is ready before root number ri runs.
+  bool early(int b, size_t ri, const std::map<int, size_t> &ready) const {
+    if (prog.bufs[b].role == BufRole::Param) return true;
+    const auto it = ready.find(b);
+    return it != ready.end() && it->second < ri && !tail_member.count(plan.roots[it->second]);
+  }
+  // Code that stores reduction t's total `x` and its tail's values, for one
+  // thread; their buffers join the kernel's parameters.
+  std::string store_total(int t, const std::string &x, Params &p) {
+    const int out = buf_of[t];
+    const std::string so = std::to_string(out);
+    std::string c = "{ const " + std::string(dt_ctype(g.ts[t].dt)) + " r" + so + " = " + x + "; b" + so + "[0] = r" + so + ";";
+    std::set<int> mine = {out};
+    const auto it = tails.find(t);
+    if (it != tails.end())
+      for (int m : it->second) {
+        const ElemFn f = gen.element_fn("f_" + std::to_string(g.ts[m].id), m, true, true);
+        src << f.code;
+        for (const auto *v : {&f.ident, &f.ptrs})
+          for (int b : *v)
+            if (!mine.count(b) && std::find(p.in.begin(), p.in.end(), b) == p.in.end()) p.in.push_back(b);
+        const int mo = buf_of[m];
+        const std::string sm = std::to_string(mo);
+        c += " const " + std::string(dt_ctype(g.ts[m].dt)) + " r" + sm + " = " + f.call("0", [&](int b) {
+          return mine.count(b) ? "r" + std::to_string(b) : "b" + std::to_string(b) + "[0]";
+        }) + "; b" + sm + "[0] = r" + sm + ";";
+        p.out.push_back(mo);
+        mine.insert(mo);
+      }
+    return c + " }";
+  }
+
   std::vector<int> lower_reduce(int t) {
     const TNode &n = g.ts[t];
     const TNode &s = g.ts[n.a];
@@ -2113,6 +2189,8 @@ struct Lowering {
         p.in.push_back(from);
         if (flagged) p.in.push_back(flags);
         p.out.push_back(to);
+        const std::string store = final ? store_total(t, cmb + "(" + ini + "(), t)", p)
+                                        : "b" + std::to_string(to) + "[blockIdx.x] = t;";
         std::vector<int> args;
         std::string params = param_list(p, args);
         const std::string P = "b" + std::to_string(from), F = "b" + std::to_string(flags);
@@ -2142,7 +2220,7 @@ struct Lowering {
           << "  if (threadIdx.x == 0) {\n"
           << "    " << T << " t = " << ini << "();\n    bool th = false;\n"
           << "    for (int w = 0; w < 4; w++) if (whas[w]) { t = th ? " << cmb << "(t, wpart[w]) : wpart[w]; th = true; }\n"
-          << "    b" << to << "[blockIdx.x] = " << (final ? cmb + "(" + ini + "(), t)" : "t") << ";\n"
+          << "    " << store << "\n"
           << "  }\n"
           << "}\n";
         src << k.str();
@@ -2164,6 +2242,7 @@ struct Lowering {
         p.in.push_back(in);
         p.in.push_back(flags);
         p.out.push_back(out);
+        const std::string store = store_total(t, cmb + "(" + ini + "(), t)", p);
         std::vector<int> args;
         std::string params = param_list(p, args);
         const int64_t K = cdiv(np, 1024), CH = std::min<int64_t>(16, K);
@@ -2194,7 +2273,7 @@ struct Lowering {
           << "    " << T << " t = " << ini << "();\n"
           << "    bool th = false;\n"
           << "    for (int w = 0; w < 16; w++) if (whas[w]) { t = th ? " << cmb << "(t, wpart[w]) : wpart[w]; th = true; }\n"
-          << "    b" << out << "[0] = " << cmb << "(" << ini << "(), t);\n"
+          << "    " << store << "\n"
           << "  }\n"
           << "}\n";
         src << k.str();
@@ -2369,8 +2448,14 @@ struct Lowering {
     // boundary makes the partials visible: no per-workgroup release (on a
     // multi-XCD device an agent-scope release writes back the L2) and no
     // counter to reset.
-    int64_t unit = vec ? 4096 : 1024;
-    int64_t G = std::max<int64_t>(1, std::min<int64_t>(cdiv(2048, rows), cdiv(len, 4096)));
+    // A long element function (48 lines, as for the folds in maps) over too
+    // few elements for 1024 such workgroups takes an element a thread at a
+    // time instead of four: its work, not its loads, is what each
+    // workgroup's time is, and it is spread over up to 2048 of them (the
+    // one-step pricer over 100000 paths, 25 workgroups: 7.4 us, 391: 3.3).
+    const bool spread = std::count(f.code.begin(), f.code.end(), '\n') >= 48 && rows * len < (int64_t(4) << 20);
+    int64_t unit = spread ? 256 : vec ? 4096 : 1024;
+    int64_t G = std::max<int64_t>(1, std::min<int64_t>(cdiv(2048, rows), cdiv(len, spread ? 256 : 4096)));
     int64_t chunk = cdiv(cdiv(len, G), unit) * unit;
     G = cdiv(len, chunk);
     int part = add_buf("t" + id + "_partials", n.dt, rows * G, BufRole::Scratch);
@@ -2392,8 +2477,15 @@ struct Lowering {
         << "  const int lo = g * " << chunk << ";\n"
         << "  const int hi = min(lo + " << chunk << ", " << len << ");\n"
         << "  " << T << " acc = " << ini << "();\n"
-        << "  bool has = false;\n"
-        << fold_loop("lo", "hi") << block_reduce << "  if (threadIdx.x == 0) {\n"
+        << "  bool has = false;\n";
+      if (spread)
+        k << "  for (int j = lo + (int)threadIdx.x; j < hi; j += 256) {\n"
+          << "    const int i = base + j;\n"
+          << "    " << fold_in(cmb, T, f.call_scalar("i")) << "\n"
+          << "  }\n";
+      else
+        k << fold_loop("lo", "hi");
+      k << block_reduce << "  if (threadIdx.x == 0) {\n"
         << wave_parts  // every chunk is non-empty, so th holds
         << "    b" << part << "[blockIdx.x] = t;\n"
         << "  }\n"
@@ -2405,6 +2497,8 @@ struct Lowering {
       Params p;
       p.in.push_back(part);
       p.out.push_back(out);
+      const std::string total = cmb + "(" + ini + "(), t)";
+      const std::string store = rows == 1 ? store_total(t, total, p) : "b" + std::to_string(out) + "[r] = " + total + ";";
       std::vector<int> args;
       std::string params = param_list(p, args);
       std::ostringstream k;
@@ -2418,7 +2512,7 @@ struct Lowering {
         << "    for (int q = threadIdx.x; q < " << G << "; q += 256) " << fold_in(cmb, T, "b" + std::to_string(part) + "[r * " + std::to_string(G) + " + q]") << "\n"
         << block_reduce << "    if (threadIdx.x == 0) {\n"
         << wave_parts
-        << "      b" << out << "[r] = " << cmb << "(" << ini << "(), t);\n"
+        << "      " << store << "\n"
         << "    }\n"
         << "    __syncthreads();\n"
         << "  }\n"
@@ -5801,6 +5895,7 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     }
     find_sibling_groups();
     find_rowlast_gathers();
+    find_tails();
     // the side buffers are computed buffers too: allocated with the others
     // for the program's lifetime
     for (size_t b = ncomputed; b < prog.bufs.size(); b++)
@@ -5813,6 +5908,8 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
       std::vector<int> ks;
       if (sib_member.count(r)) {
         // lowered with its group's lead
+      } else if (tail_member.count(r)) {
+        // computed by its reduction's last kernel
       } else if (sib_lead.count(r)) {
         const int sc = sib_lead[r];
         ks = lower_scan(sc, sib_reds[sc]);

@@ -206,4 +206,8 @@ size_t noalloc_scratch_spare();
 void *noalloc_scratch(int device);
 void noalloc_scratch_clear(void *base, size_t bytes, void *stream);
 
+// Copies `bytes` (a multiple of 16, below 2^31) between device memory and
+// pinned host memory with a kernel on `stream`.
+void stage_copy(void *dst, const void *src, size_t bytes, void *stream);
+
 }  // namespace cchip

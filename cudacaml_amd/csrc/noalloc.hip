@@ -1,5 +1,6 @@
-// The static scratch of the allocation-free entry point
-// (cchip_program_run_resident_noalloc, backend.cpp).
+// The library's own device code: the static scratch of the allocation-free
+// entry point (cchip_program_run_resident_noalloc, backend.cpp), the kernel
+// that clears it, and the copy of a synchronous run's small values.
 //
 // Template scratch (look-back status words and tile counters, split
 // reduction partials, scatter counts, offsets and staged pairs, split-k
@@ -33,6 +34,12 @@ namespace {
 __global__ __launch_bounds__(256) void cchip_scratch_clear(uint4 *__restrict__ p, size_t n16) {
   const uint4 z = make_uint4(0u, 0u, 0u, 0u);
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) p[i] = z;
+}
+
+// A synchronous run's small values between the executor's device block and
+// its pinned host block, either way.
+__global__ __launch_bounds__(256) void cchip_stage_copy(uint4 *__restrict__ dst, const uint4 *__restrict__ src, int n16) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n16; i += gridDim.x * 256) dst[i] = src[i];
 }
 
 constexpr int kMaxDevices = 64;
@@ -74,6 +81,15 @@ void noalloc_scratch_clear(void *base, size_t bytes, void *stream) {
   void *args[] = {&p, &n16};
   check_hip(hipLaunchKernel((const void *)cchip_scratch_clear, dim3(grid), dim3(256), args, 0, (hipStream_t)stream),
             "hipLaunchKernel(scratch clear)");
+}
+
+void stage_copy(void *dst, const void *src, size_t bytes, void *stream) {
+  uint4 *d = (uint4 *)dst;
+  const uint4 *f = (const uint4 *)src;
+  int n16 = (int)(bytes / 16);
+  void *args[] = {&d, &f, &n16};
+  check_hip(hipLaunchKernel((const void *)cchip_stage_copy, dim3((n16 + 255) / 256), dim3(256), args, 0, (hipStream_t)stream),
+            "hipLaunchKernel(stage copy)");
 }
 
 }  // namespace cchip

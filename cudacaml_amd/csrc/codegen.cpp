@@ -1256,6 +1256,9 @@ struct Lowering {
   // their kernel (set by lower_program for a second lowering): their
   // kernels store nothing but the partials, and their buffers are elided.
   std::set<int> no_store;
+  // Whether matrix products may split k, and the scratch they took for it.
+  bool ksplit = true;
+  int64_t ksplit_bytes = 0;
   // Row roots over one tensor fused into one kernel: a row scan that takes
   // the one-workgroup-a-row tile template, and the reductions of the same
   // tensor's rows that fold as a tree. The group's first root in the plan
@@ -5023,6 +5026,30 @@ struct Lowering {
     }
     return cdiv(M, 128) * cdiv(N, 128) < 208 && tune("mm_split", 1) != 2 ? 64 : 128;
   }
+  // Partial products a grid of few tiles splits k into: a tile's k loop is
+  // a chain of loads, LDS and matrix instructions, and CUs without a tile
+  // idle through all of it. The parts cost a write, a read and a kernel, so
+  // there are three or more (two, where tiles of 64x64 f64 would leave 256
+  // CUs a round and a bit), and slices stay 128 deep for up to a workgroup
+  // a CU, 256 for two (f64: 192 for four of its small ones; past 128 tiles
+  // only from K = 768). Unsplit / split, us a product with its launches:
+  // f32 64x64x512 13.6 / 8.7, 64x64x4096 97 / 8.5, 512^3 14.0 / 9.2,
+  // 512x512x2048 49 / 18, 700x901x1500 39 / 29 (and in two: 900x1000x512
+  // 14.8 / 18.5); f64 64x64x2048 34 / 8.5, 100x200x700 14.8 / 8.9,
+  // 512x512x1024 21.8 / 18.8 (512x512x576 10.5 / 15.8), 1500x1101x2001 in
+  // two 164 / 135 (1400x1400x2000, 484 tiles, 121 / 133). The sums are
+  // shorter: f64 64x64x2048 1.5e-15 off the exact product, split 5.1e-16.
+  int64_t mfma_ksplit(DT dt, int64_t M, int64_t N, int64_t K) const {
+    if (!ksplit || !tune("mm_ksplit", 1)) return 1;
+    const int64_t BM = mfma_bm(dt, M, N), tiles = cdiv(M, BM) * cdiv(N, BM);
+    if (dt == DT::F64) {
+      if (tiles > (BM == 64 ? 448 : 1024) || (tiles > 128 && K < 768)) return 1;
+      const int64_t G = std::min<int64_t>({1024 / tiles, K / 192, 32});
+      return G >= (BM == 64 ? 2 : 3) ? G : 1;
+    }
+    const int64_t G = std::min<int64_t>(32, std::max(std::min(256 / tiles, K / 128), std::min(512 / tiles, K / 256)));
+    return G >= 3 ? G : 1;
+  }
   // Byte offsets into the operands, the rows past their ends included, are
   // 32-bit in the ragged form.
   static bool mfma_fits(DT dt, int64_t M, int64_t N, int64_t K) {
@@ -5189,9 +5216,6 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
         if (!dup) p.in.push_back(o->buf);
       }
     }
-    p.out.push_back(out);
-    std::vector<int> args;
-    std::string params = param_list(p, args);
     const int64_t ALDS = A.kcontig ? BM * KP : BK * MP;
     const int64_t BLDS = B.kcontig ? BM * KP : BK * MP;
     std::string V = f64 ? "cc_v2<double>" : "cc_v4<float>";  // one 16-byte access
@@ -5302,6 +5326,12 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     std::string mfma = f64 ? "__builtin_amdgcn_mfma_f64_16x16x4f64" : "__builtin_amdgcn_mfma_f32_32x32x2f32";
     int64_t tiles_m = cdiv(M, BM), tiles_n = cdiv(N, BM), ntiles = tiles_m * tiles_n;
     const int64_t nk = cdiv(K, BK);
+    // Small grids split k (mfma_ksplit): workgroup (ks, tile) sums k tiles
+    // [ks * KS, ks * KS + KS) of its tile into partial product ks.
+    const int64_t KS = split ? nk : cdiv(nk, mfma_ksplit(n.dt, M, N, K)), KG = cdiv(nk, KS);
+    const bool parts = KG > 1;
+    const int dst = parts ? add_buf("t" + id + "_kpart", n.dt, KG * M * N, BufRole::Scratch) : out;
+    if (parts) ksplit_bytes += (prog.bufs[dst].bytes() + 255) & ~int64_t(255);
     // f64: one LDS buffer, refilled between two barriers (the fragments are
     // in registers by the first), and a four-waves-a-SIMD register budget,
     // which also keeps the accumulators in ordinary vector registers: at
@@ -5310,6 +5340,9 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     // from either.
     const bool single = f64 && tune("mm_f64_single", 1) != 0;
     const int64_t waves = f64 && BM == 64 ? std::max<int64_t>(0, std::min<int64_t>(8, tune("mm_f64_waves", 4))) : 0;
+    p.out.push_back(dst);
+    std::vector<int> args;
+    std::string params = param_list(p, args);
     k << "typedef " << T << " " << accT << " __attribute__((ext_vector_type(" << NACC << ")));\n"
       << "extern \"C\" __global__ __launch_bounds__(256) ";
     if (waves > 0) k << "__attribute__((amdgpu_waves_per_eu(" << waves << ", " << waves << "))) ";
@@ -5330,6 +5363,8 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
       // blocks are dispatched round-robin over the 8 XCDs; give each XCD a
       // contiguous run of tiles so its L2 sees shared A row panels.
       << "  int tile = blockIdx.x;\n";
+    // partial by partial, so that an XCD's run of tiles shares one k range
+    if (parts) k << "  const int ks = tile / " << ntiles << ";\n  tile -= ks * " << ntiles << ";\n";
     if (ntiles % 8 != 0 && ntiles > 8)
       k << "  { const int x = tile % 8; tile = x * " << ntiles / 8 << " + (x < " << ntiles % 8 << " ? x : " << ntiles % 8
         << ") + tile / 8; }\n";
@@ -5514,20 +5549,25 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     // about 1.7e-4 for one f32 accumulator (and for the interpreter's own
     // sequential sum). KC = mm_chunk_k, 256 by default.
     int64_t KCT = f64 ? 0 : std::max<int64_t>(0, tune("mm_chunk_k", 256) / BK);
-    if (KCT >= nk) KCT = 0;  // one chunk: nothing to fold
+    if (KCT >= KS) KCT = 0;  // one chunk: nothing to fold
+    const std::string k1 = parts ? "k1" : std::to_string(nk), it0 = parts ? "it - k0" : "it";
     if (KCT > 0)
       k << "  " << accT << " tot[" << RT << "][" << RT << "];\n"
         << "#pragma unroll\n"
         << "  for (int i = 0; i < " << RT << "; i++)\n"
         << "#pragma unroll\n"
         << "    for (int j = 0; j < " << RT << "; j++) tot[i][j] = (" << accT << ")(0);\n";
-    k << "  int kt = 0;\n"
-      << gload(A, true, "ra") << gload(B, false, "rb") << lstore(A, "As[0]", "ra") << lstore(B, "Bs[0]", "rb")
+    if (parts)
+      k << "  const int k0 = ks * " << KS << ", k1 = min(k0 + " << KS << ", " << nk << ");\n"
+        << "  int kt = k0 * " << BK << ";\n";
+    else
+      k << "  int kt = 0;\n";
+    k << gload(A, true, "ra") << gload(B, false, "rb") << lstore(A, "As[0]", "ra") << lstore(B, "Bs[0]", "rb")
       << "  __syncthreads();\n"
-      << "  for (int it = 0; it < " << nk << "; it++) {\n"
-      << "    const int buf = " << (single ? "0" : "it & 1") << ";\n"
+      << "  for (int it = " << (parts ? "k0" : "0") << "; it < " << k1 << "; it++) {\n"
+      << "    const int buf = " << (single ? "0" : "(" + it0 + ") & 1") << ";\n"
       << "    kt = (it + 1) * " << BK << ";\n"
-      << "    if (it + 1 < " << nk << ") {\n"
+      << "    if (it + 1 < " << k1 << ") {\n"
       << gload(A, true, "ra") << gload(B, false, "rb") << "    }\n"
       // keeps the scheduler from sinking the next tile's loads to their
       // LDS stores (to save registers), which left them unhidden
@@ -5539,7 +5579,7 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
       << fragload(A, "al", "fa", "wm") << fragload(B, "bl", "fb", "wn");
     if (single)  // every wave holds its fragments: the buffer takes the next tile
       k << "      __syncthreads();\n"
-        << "      if (it + 1 < " << nk << ") {\n"
+        << "      if (it + 1 < " << k1 << ") {\n"
         << lstore(A, "As[0]", "ra") << lstore(B, "Bs[0]", "rb") << "      }\n";
     k << "#pragma unroll\n"
       << "      for (int s2 = 0; s2 < " << S << "; s2++)\n"
@@ -5550,10 +5590,10 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
       << "(fa[i][s2], fb[j][s2], acc[i][j], 0, 0, 0);\n"
       << "    }\n";
     if (!single)
-      k << "    if (it + 1 < " << nk << ") {\n"
+      k << "    if (it + 1 < " << k1 << ") {\n"
         << lstore(A, "As[buf ^ 1]", "ra") << lstore(B, "Bs[buf ^ 1]", "rb") << "    }\n";
     if (KCT > 0)
-      k << "    if ((it + 1) % " << KCT << " == 0" << (nk % KCT != 0 ? " || it + 1 == " + std::to_string(nk) : "") << ") {\n"
+      k << "    if ((" << it0 << " + 1) % " << KCT << " == 0" << (parts || nk % KCT != 0 ? " || it + 1 == " + k1 : "") << ") {\n"
         << "#pragma unroll\n"
         << "      for (int i = 0; i < " << RT << "; i++)\n"
         << "#pragma unroll\n"
@@ -5575,14 +5615,31 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
       k << "        const int row = bm + wm + i * 32 + (r / 4) * 8 + (lane / 32) * 4 + (r % 4);\n";
     k << "        ";
     if (ragged) k << "if (row < " << M << " && col < " << N << ") ";
-    k << "b" << out << "[(size_t)row * " << N << " + col] = " << (KCT > 0 ? "tot" : "acc") << "[i][j][r];\n"
+    k << "b" << dst << "[" << (parts ? "(size_t)ks * " + std::to_string(M * N) + " + " : "") << "(size_t)row * " << N
+      << " + col] = " << (KCT > 0 ? "tot" : "acc") << "[i][j][r];\n"
       << "      }\n"
       << "    }\n"
       << "}\n";
+    // the partial products added in order of k, all of an element's loads in
+    // flight
+    if (parts)
+      k << "extern \"C\" __global__ __launch_bounds__(256) void " << kname << "_ksum(const " << T << "* __restrict__ b" << dst
+        << ", " << T << "* __restrict__ b" << out << ") {\n"
+        << "  const int q = blockIdx.x * 256 + threadIdx.x;\n"
+        << "  if (q >= " << M * N << ") return;\n"
+        << "  " << T << " v[" << KG << "];\n"
+        << "#pragma unroll\n"
+        << "  for (int s = 0; s < " << KG << "; s++) v[s] = b" << dst << "[(size_t)s * " << M * N << " + q];\n"
+        << "#pragma unroll\n"
+        << "  for (int s = 1; s < " << KG << "; s++) v[0] = v[0] + v[s];\n"
+        << "  b" << out << "[q] = v[0];\n"
+        << "}\n";
     src << k.str();
     std::string role = std::string("matmul_mfma_") + (f64 ? "f64" : "f32") + "_" + "a" + std::to_string(A.mode) +
                        "b" + std::to_string(B.mode);
-    return {add_kernel(kname, args, (int)ntiles, 256, role)};
+    std::vector<int> ks = {add_kernel(kname, args, (int)(ntiles * KG), 256, role)};
+    if (parts) ks.push_back(add_kernel(kname + "_ksum", {dst, out}, (int)cdiv(M * N, 256), 256, "matmul_ksum"));
+    return ks;
   }
 
   // ---- Skinny matmul: split over k ------------------------------------------
@@ -5969,9 +6026,11 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
 
 int64_t tune_knob(const char *key, int64_t dflt) { return tune(key, dflt); }
 
-ProgramIR lower_program(const Graph &g) {
+static ProgramIR lower_program(const Graph &g, bool ksplit, int64_t *ksplit_bytes) {
   Lowering l(g);
+  l.ksplit = ksplit;
   l.run();
+  *ksplit_bytes = l.ksplit_bytes;
   // A map root whose reduction folds in its kernel may have no reader
   // left: a tensor materialised because the reduction's expression uses it
   // twice (config 5's last adjoint map, 1 GiB). Lowered again, its kernel
@@ -5993,11 +6052,25 @@ ProgramIR lower_program(const Graph &g) {
     if (!unread.empty()) {
       Lowering l2(g);
       l2.no_store = unread;
+      l2.ksplit = ksplit;
       l2.run();
       return l2.prog;
     }
   }
   return l.prog;
+}
+
+ProgramIR lower_program(const Graph &g) {
+  int64_t extra = 0, scratch = 256;
+  ProgramIR p = lower_program(g, true, &extra);
+  // A program that fits the allocation-free scratch without the partial
+  // products of its matrix products, and not with them, goes without.
+  for (const BufSpec &b : p.bufs)
+    if (b.role == BufRole::Scratch) scratch += (std::max<int64_t>(b.bytes(), 1) + 255) & ~int64_t(255);
+  const int64_t cap = (int64_t)noalloc_scratch_capacity();
+  if (extra && scratch > cap && scratch - extra <= cap + (int64_t)noalloc_scratch_spare())
+    return lower_program(g, false, &extra);
+  return p;
 }
 
 std::string plan_to_string(const ProgramIR &p) {

@@ -2532,7 +2532,7 @@ struct Lowering {
   struct TileShape {
     int64_t GW, NW, U, SL, tile, tpr;  // GW: elements a thread takes of a slice
   };
-  static TileShape tile_shape(int64_t len, DT dt) {
+  static TileShape tile_shape(int64_t len, DT dt, int64_t rows = 1) {
     const bool wide = dt_size(dt) == 8;
     auto shape = [&](int64_t NW, int64_t GW) {
       TileShape s;
@@ -2552,8 +2552,10 @@ struct Lowering {
     // wave's access is one contiguous run: 4 elements of 8 bytes would be
     // two 16-byte accesses 32 bytes apart, each half of every line (2^27
     // f64: 463 -> 432 us). One-tile rows keep 4, with half the slices to
-    // scan (1500 x 3001 f64: 16.0 us, 17.2 with 2).
-    return wide && one.tpr > 1 ? shape(NW, 2) : one;
+    // scan (1500 x 3001 f64: 16.0 us, 17.2 with 2), and so do rows of up to
+    // 16 of those tiles: smaller ones only lengthen their chains (100 x
+    // 32768 f64: 27 us in two tiles a row, 34 in three).
+    return wide && one.tpr > (rows > 1 ? 16 : 1) ? shape(NW, 2) : one;
   }
 
   // Whether a scan root takes the tile template with one tile a row (one
@@ -2807,7 +2809,7 @@ struct Lowering {
     // 12, 14, 15 and 16 slices. 8-byte values over 12 slices of 1024: 2^27
     // i64 or f64 in 432 us (14 and 16 slices: 460 and 434, the latter
     // spilling).
-    TileShape ts = tile_shape(len, n.dt);
+    TileShape ts = tile_shape(len, n.dt, rows);
     const int GW = (int)ts.GW;
     // A whole-tensor scan whose input stays in the 256 MB MALL between two
     // reads takes two passes instead of the look-back: every tile's total
@@ -2826,7 +2828,9 @@ struct Lowering {
     // Short chains of tiles take fewer slices a tile, for 256 tiles or
     // more: one CU's load of a large tile is what they wait for (100000
     // i32: 12.7 us in 26624-element tiles, 7.7 in 4096; 1M f64 14.7 / 12).
-    if (ts.tpr > 1) {
+    // Rows of 8-byte values only below 64 tiles (30 x 60000 f64: 22.5 us in
+    // 120 tiles, 24.3 in 270; 8 x 20000 in 16 tiles 17.5, in 80 15.9).
+    if (ts.tpr > 1 && !(wide && rows > 1 && rows * ts.tpr >= 64)) {
       const int64_t u = two_pass ? 4 : std::max<int64_t>(2, cdiv(rows * len, ts.SL * 256));
       if (u < ts.U) {
         ts.U = u;

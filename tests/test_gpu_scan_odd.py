@@ -72,7 +72,7 @@ def test_one_tile_a_row(device, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", [F32, F64, I32, I64], ids=lambda d: d.name)
-@pytest.mark.parametrize("shape", [(3, 26625), (2, 26627), (2, 40001), (5, 300001), (50003,), (1 << 20,)], ids=str)
+@pytest.mark.parametrize("shape", [(3, 26625), (2, 26627), (2, 40001), (5, 300001), (70, 27001), (50003,), (1 << 20,)], ids=str)
 def test_look_back(device, dtype, shape):
     assert "scan_lookback" in templates(graph(dtype, shape, D.add, 0))
     check(dtype, shape, D.add, 2, shape[-1])

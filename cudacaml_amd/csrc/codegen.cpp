@@ -2552,10 +2552,10 @@ struct Lowering {
     // wave's access is one contiguous run: 4 elements of 8 bytes would be
     // two 16-byte accesses 32 bytes apart, each half of every line (2^27
     // f64: 463 -> 432 us). One-tile rows keep 4, with half the slices to
-    // scan (1500 x 3001 f64: 16.0 us, 17.2 with 2), and so do rows of up to
-    // 16 of those tiles: smaller ones only lengthen their chains (100 x
-    // 32768 f64: 27 us in two tiles a row, 34 in three).
-    return wide && one.tpr > (rows > 1 ? 16 : 1) ? shape(NW, 2) : one;
+    // scan (1500 x 3001 f64: 16.0 us, 17.2 with 2), and so do
+    // several rows: smaller tiles lengthen their chains (100 x 32768 f64: 27
+    // us in two tiles a row, 34 in three; 16 x 500000 48 and 57).
+    return wide && rows == 1 && one.tpr > 1 ? shape(NW, 2) : one;
   }
 
   // Whether a scan root takes the tile template with one tile a row (one

@@ -58,8 +58,6 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 FP32_MFMA_TFLOPS = 157.3
 FP64_MFMA_TFLOPS = 78.6
-# f32 products in three bf16 planes an operand: six bf16 products each
-SPLIT_MFMA_TFLOPS = 2516.6 / 6
 
 
 def log(*a):
@@ -432,7 +430,7 @@ def counter_passes(config):
         passes.append(list(VALU_CLASSES) + ["GRBM_GUI_ACTIVE"])
     if config in MFMA_CONFIGS:
         passes.append(["SQ_VALU_MFMA_BUSY_CYCLES", "SQ_INSTS_VALU_MFMA_MOPS_F32", "SQ_INSTS_VALU_MFMA_MOPS_F64",
-                       "SQ_INSTS_VALU_MFMA_MOPS_BF16", "GRBM_GUI_ACTIVE"])
+                       "GRBM_GUI_ACTIVE"])
     return passes
 
 
@@ -676,10 +674,9 @@ def main():
         uid = int(dom.split("_")[1])
         mm = [t for g, _, _, _ in w.programs for t in g.order if t.uid == uid][0]
         fl = 2 * mm.shape[0] * mm.shape[1] * mm.a.shape[1]
-        split = any("cc_split4" in H.source(g) for g, _, _, _ in w.programs if mm in g.order)
-        peak = FP64_MFMA_TFLOPS if mm.dtype.name == "f64" else SPLIT_MFMA_TFLOPS if split else FP32_MFMA_TFLOPS
+        peak = FP64_MFMA_TFLOPS if mm.dtype.name == "f64" else FP32_MFMA_TFLOPS
         achieved = fl / (dom_avg_ms * 1e-3) / 1e12
-        roof = {"bound": "mfma", "achieved": round(achieved, 2), "peak": round(peak, 1), "unit": "TFLOP/s",
+        roof = {"bound": "mfma", "achieved": round(achieved, 2), "peak": peak, "unit": "TFLOP/s",
                 "frac": round(achieved / peak, 4), "traffic": traffic, "flops_per_launch": fl}
     else:
         achieved = dom_bytes / (dom_avg_ms * 1e-3) / 1e9
@@ -727,8 +724,7 @@ def main():
         # counted (512 flops per MOPS unit) per clock against the peak per
         # clock, both from one pass.
         cycles = dc["GRBM_GUI_ACTIVE"] / XCC_COUNT
-        mops = (dc.get("SQ_INSTS_VALU_MFMA_MOPS_F32", 0.0) + dc.get("SQ_INSTS_VALU_MFMA_MOPS_F64", 0.0)
-                + dc.get("SQ_INSTS_VALU_MFMA_MOPS_BF16", 0.0) / 6)
+        mops = dc.get("SQ_INSTS_VALU_MFMA_MOPS_F32", 0.0) + dc.get("SQ_INSTS_VALU_MFMA_MOPS_F64", 0.0)
         cflops = mops * 512
         peak_tf = roof["peak"]
         roof["mfma"] = {"busy_frac": round(dc["SQ_VALU_MFMA_BUSY_CYCLES"] / (simds * cycles), 4),
@@ -737,7 +733,7 @@ def main():
                         "frac_per_clock": round(cflops / cycles / (peak_tf * 1e12 / MFMA_CLOCK_HZ), 4),
                         "clock_ghz_implied": round(cycles / (dom_avg_ms * 1e-3) / 1e9, 3),
                         "how": "busy = SQ_VALU_MFMA_BUSY_CYCLES / (SIMDs x GRBM_GUI_ACTIVE/8); flops = 512 x "
-                               "SQ_INSTS_VALU_MFMA_MOPS_F32/F64, BF16 by six; frac_per_clock against peak / 2.4 GHz; one pass"}
+                               "SQ_INSTS_VALU_MFMA_MOPS_F32/F64; frac_per_clock against peak / 2.4 GHz; one pass"}
     roof["kernel"] = dom
     roof["template"] = dom_role
     roof["algorithmic_bytes"] = dom_bytes

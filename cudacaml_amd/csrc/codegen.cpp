@@ -5028,7 +5028,7 @@ struct Lowering {
       if (want > 0) return want == 128 || want == 32 ? want : 64;
       return cdiv(M, 64) * cdiv(N, 64) < 300 ? 32 : 64;
     }
-    return cdiv(M, 128) * cdiv(N, 128) < 208 && tune("mm_split", 1) != 2 ? 64 : 128;
+    return cdiv(M, 128) * cdiv(N, 128) < 208 ? 64 : 128;
   }
   // Partial products a grid of few tiles splits k into: a tile's k loop is
   // a chain of loads, LDS and matrix instructions, and CUs without a tile
@@ -5070,78 +5070,6 @@ struct Lowering {
     return want == 64 || want == 32 ? want : 16;
   }
 
-  // ---- f32 products on the bf16 matrix cores --------------------------------
-  // gfx950 multiplies bf16 about twelve times as fast as f32 (1.5-1.8
-  // PFLOP/s against 0.15 in register-only loops). An f32 is the exact sum
-  // of three bf16 (8 + 8 + 8 bits, each the rest rounded to nearest: h, m,
-  // l), and a product of two bf16 is exact in f32, so
-  //   x y = h h' + (h m' + m h') + (h l' + m m' + l h') + rest,
-  // where the rest is at most 2^-23 and in root mean square about 2^-26 of
-  // |x y|, below the rounding of the sums themselves. A v_mfma_f32_32x32x16_
-  // bf16 rounds its accumulator twice for 16 k steps (it adds 8 exact
-  // products at a time), so the six instructions of 16 steps round it 12
-  // times where sixteen steps of v_mfma_f32_32x32x2f32 round it 16 times,
-  // and the chunked totals (mm_chunk_k) are the same: the error against the
-  // exact product is no larger (4096^3 N(0,1): 2.5e-7 against 3.0e-7
-  // normwise).
-  // The bf16 instructions cut what they shift out towards minus infinity,
-  // a mean error of -6e-8 of the result's root mean square at K = 4096
-  // where the f32 instructions have none, which a sum over the result
-  // gathers (sum of 4096^2 entries: 6e-4 off). So every other k tile is
-  // multiplied with its sign flipped, A's values and the accumulators with
-  // them, and the cuts cancel; what an odd number of tiles leaves changes
-  // sign with the parity of the row's bits.
-  // The split is exact while 2^-100 <= |x| < 2^60 or x = 0; below, l would
-  // lose bits to the smallest bf16, above, partial products could overflow
-  // to infinities of both signs. The range is tracked as tiles are split
-  // (cc_rng: the largest |x| and the smallest non-zero one) and looked at
-  // once every 8 k tiles; a tile that meets anything outside (infinities and
-  // NaN too) is computed again by the f32 instructions, in the same kernel
-  // (4096^3 with such a value early in every row panel: 1071 us against
-  // 1037 on the f32 instructions alone; one infinity in a last k tile: 1768,
-  // its 32 tiles beginning again at the end).
-  bool split_emitted = false;
-  void emit_split_helpers() {
-    if (split_emitted) return;
-    split_emitted = true;
-    src << R"SPLIT(
-typedef __bf16 cc_bf8 __attribute__((ext_vector_type(8)));
-typedef __bf16 cc_bf2 __attribute__((ext_vector_type(2)));
-typedef float cc_f2v __attribute__((ext_vector_type(2)));
-typedef cc_u32 cc_u32x2 __attribute__((ext_vector_type(2)));
-struct cc_rng { float mx; cc_u32 mn; };
-__device__ __forceinline__ bool cc_outside(const cc_rng& c) {
-  return !(c.mx < 0x1p60f) || c.mn < (27u << 24) - 1u;
-}
-__device__ __forceinline__ cc_u32 cc_bf16x2(float a, float b) {
-  const cc_f2v v = {a, b};
-  return __builtin_bit_cast(cc_u32, __builtin_convertvector(v, cc_bf2));
-}
-__device__ __forceinline__ void cc_split2(float a, float b, cc_u32& h, cc_u32& m, cc_u32& l, cc_rng& c) {
-  c.mx = __builtin_elementwise_maximum(c.mx, __builtin_elementwise_maximum(__builtin_fabsf(a), __builtin_fabsf(b)));
-  const cc_u32 ua = (__builtin_bit_cast(cc_u32, a) << 1) - 1u, ub = (__builtin_bit_cast(cc_u32, b) << 1) - 1u;
-  c.mn = __builtin_elementwise_min(c.mn, __builtin_elementwise_min(ua, ub));
-  h = cc_bf16x2(a, b);
-  const float ra = a - __builtin_bit_cast(float, h << 16), rb = b - __builtin_bit_cast(float, h & 0xffff0000u);
-  m = cc_bf16x2(ra, rb);
-  l = cc_bf16x2(ra - __builtin_bit_cast(float, m << 16), rb - __builtin_bit_cast(float, m & 0xffff0000u));
-}
-__device__ __forceinline__ float cc_sign(float x, cc_u32 s) {
-  return __builtin_bit_cast(float, __builtin_bit_cast(cc_u32, x) ^ s);
-}
-// Four values along k, their sign bits flipped by s, into the three planes
-// of a tile, P elements apart.
-__device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __bf16* p, int P, cc_rng& r, cc_u32 s) {
-  cc_u32 h0, m0, l0, h1, m1, l1;
-  cc_split2(cc_sign(a, s), cc_sign(b, s), h0, m0, l0, r);
-  cc_split2(cc_sign(c, s), cc_sign(d, s), h1, m1, l1, r);
-  *(cc_u32x2*)p = cc_u32x2{h0, h1};
-  *(cc_u32x2*)(p + P) = cc_u32x2{m0, m1};
-  *(cc_u32x2*)(p + 2 * P) = cc_u32x2{l0, l1};
-}
-)SPLIT";
-  }
-
   // ---- Matmul on the matrix cores ------------------------------------------
   // f32: v_mfma_f32_32x32x2f32, block tile 128x128x16 (64x64x64 for small
   // grids), four waves of 64x64 (32x32).
@@ -5170,9 +5098,7 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     // end of A, k rows past the end of B), and k columns past K are zeroed
     // in the last k tile. Columns past N read the next row's values; they
     // reach only outputs that are not stored.
-    const bool split = !f64 && BM == 128 && K >= 64 && tune("mm_split", 1) != 0 &&
-                       (mfma_fits(n.dt, M, N, K) || (M % BM == 0 && N % BM == 0 && K % 32 == 0));
-    const bool ragged = M % BM != 0 || N % BM != 0 || K % BK != 0 || (split && K % 32 != 0);
+    const bool ragged = M % BM != 0 || N % BM != 0 || K % BK != 0;
     const int64_t G = 64 / MT;    // lane groups along k
     const int64_t S = BK / G;     // k steps per tile held by one lane
     const int64_t WT = BM / 2;    // wave tile
@@ -5332,7 +5258,7 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     const int64_t nk = cdiv(K, BK);
     // Small grids split k (mfma_ksplit): workgroup (ks, tile) sums k tiles
     // [ks * KS, ks * KS + KS) of its tile into partial product ks.
-    const int64_t KS = split ? nk : cdiv(nk, mfma_ksplit(n.dt, M, N, K)), KG = cdiv(nk, KS);
+    const int64_t KS = cdiv(nk, mfma_ksplit(n.dt, M, N, K)), KG = cdiv(nk, KS);
     const bool parts = KG > 1;
     const int dst = parts ? add_buf("t" + id + "_kpart", n.dt, KG * M * N, BufRole::Scratch) : out;
     if (parts) ksplit_bytes += (prog.bufs[dst].bytes() + 255) & ~int64_t(255);
@@ -5350,19 +5276,10 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     k << "typedef " << T << " " << accT << " __attribute__((ext_vector_type(" << NACC << ")));\n"
       << "extern \"C\" __global__ __launch_bounds__(256) ";
     if (waves > 0) k << "__attribute__((amdgpu_waves_per_eu(" << waves << ", " << waves << "))) ";
-    if (split) k << "__attribute__((amdgpu_waves_per_eu(2, 2))) ";
-    k << "void " << kname << "(" << params << ") {\n";
-    if (split) {
-      emit_split_helpers();
-      k << "  __shared__ __attribute__((aligned(16))) char lds[" << std::max<int64_t>(2 * 4 * (ALDS + BLDS), 2 * 3 * 2 * BM * 40)
-        << "];\n"
-        << "  float (*As)[" << ALDS << "] = (float (*)[" << ALDS << "])lds;\n"
-        << "  float (*Bs)[" << BLDS << "] = (float (*)[" << BLDS << "])(lds + " << 2 * 4 * ALDS << ");\n";
-    } else {
-      k << "  __shared__ __attribute__((aligned(16))) " << T << " As[" << (single ? 1 : 2) << "][" << ALDS << "];\n"
-        << "  __shared__ __attribute__((aligned(16))) " << T << " Bs[" << (single ? 1 : 2) << "][" << BLDS << "];\n";
-    }
-    k << "  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;\n"
+    k << "void " << kname << "(" << params << ") {\n"
+      << "  __shared__ __attribute__((aligned(16))) " << T << " As[" << (single ? 1 : 2) << "][" << ALDS << "];\n"
+      << "  __shared__ __attribute__((aligned(16))) " << T << " Bs[" << (single ? 1 : 2) << "][" << BLDS << "];\n"
+      << "  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;\n"
       << "  const int wm = (wid >> 1) * " << WT << ", wn = (wid & 1) * " << WT << ";\n"
       // blocks are dispatched round-robin over the 8 XCDs; give each XCD a
       // contiguous run of tiles so its L2 sees shared A row panels.
@@ -5388,157 +5305,6 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
         if (o->mode != 2)
           k << "  const __amdgpu_buffer_rsrc_t " << (o == &A ? "qa" : "qb") << " = cc_rsrc(b" << o->buf << ", "
             << prog.bufs[o->buf].bytes() << "u);\n";
-    if (split) {
-      // Tiles of 128 x 128 x 32, three bf16 planes an operand, rows of 40
-      // (32 and a pad that spreads the 16-byte fragment reads over the LDS
-      // banks). A thread stages 4 x 4 elements of each operand: four k of
-      // four rows where k is contiguous in memory, else four k rows of four
-      // columns. 61 KB of LDS and 216 VGPRs: two workgroups a CU, one
-      // splitting while the other multiplies. 4096^3: 1037 us on the f32
-      // instructions, 750-785 so (175-183 TFLOP/s; 1.1 PFLOP/s of bf16, what
-      // the vendor library's bf16 8192^3 runs at on the same card). Two LDS
-      // buffers of 16 k, or the split moved between the multiplies,
-      // measured the same and slower (769, 2057 with spills).
-      const std::string MM = "__builtin_amdgcn_mfma_f32_32x32x16_bf16";
-      auto sload = [&](const Opnd &o, bool is_a, const std::string &reg) {
-        std::ostringstream l;
-        const std::string mnb = is_a ? "bm" : "bn", q = is_a ? "qa" : "qb";
-        const int64_t MNtot = is_a ? M : N;
-        const bool rows = o.mode == 2 ? is_a : o.kcontig;
-        l << "#pragma unroll\n"
-          << "      for (int i = 0; i < 4; i++) {\n";
-        if (rows)
-          l << "        const int mn = " << mnb << " + lr + 32 * i, kk = kt + lk * 4;\n";
-        else
-          l << "        const int mn = " << mnb << " + lr * 4, kk = kt + lk * 4 + i;\n";
-        if (o.mode == 2) {
-          for (int c = 0; c < 4; c++) {
-            const std::string m = rows ? "mn" : strf("(mn + %d)", c), kc = rows ? strf("(kk + %d)", c) : "kk";
-            const std::string idx = is_a ? m + " * " + std::to_string(K) + " + " + kc
-                                         : kc + " * " + std::to_string(N) + " + " + m;
-            l << "        " << reg << "[i][" << c << "] = ";
-            if (ragged) l << "(" << m << " < " << MNtot << " && " << kc << " < " << K << ") ? ";
-            l << o.fn.call_scalar(idx) << (ragged ? " : 0.0f;\n" : ";\n");
-          }
-        } else {
-          const std::string e = rows ? "mn * " + std::to_string(K) + " + kk" : "kk * " + std::to_string(MNtot) + " + mn";
-          if (ragged) {
-            l << "        " << reg << "[i] = cc_bldv<cc_f4v>(" << q << ", (" << e << ") * 4);\n";
-            if (rows && K % 32 != 0) {
-              l << "        if (kt > " << K - 32 << ") {\n";
-              for (int c = 0; c < 4; c++)
-                l << "          if (kk + " << c << " >= " << K << ") " << reg << "[i][" << c << "] = 0.0f;\n";
-              l << "        }\n";
-            }
-          } else {
-            l << "        " << reg << "[i] = *(const cc_f4v*)(b" << o.buf << " + (size_t)"
-              << (rows ? "mn * " + std::to_string(K) + " + kk" : "kk * " + std::to_string(MNtot) + " + mn") << ");\n";
-          }
-        }
-        l << "      }\n";
-        return l.str();
-      };
-      auto sstore = [&](const Opnd &o, bool is_a, const std::string &reg, const std::string &lds) {
-        const bool rows = o.mode == 2 ? is_a : o.kcontig;
-        std::ostringstream l;
-        l << "#pragma unroll\n"
-          << "      for (int i = 0; i < 4; i++) cc_split4(";
-        if (rows)
-          l << reg << "[i][0], " << reg << "[i][1], " << reg << "[i][2], " << reg << "[i][3], " << lds
-            << " + (lr + 32 * i) * 40 + lk * 4";
-        else
-          l << reg << "[0][i], " << reg << "[1][i], " << reg << "[2][i], " << reg << "[3][i], " << lds
-            << " + (lr * 4 + i) * 40 + lk * 4";
-        l << ", " << 128 * 40 << ", rng, ";
-        if (is_a)
-          l << "((cc_u32)__builtin_popcount(" << (rows ? "bm + lr + 32 * i" : "bm + lr * 4 + i") << ") + (cc_u32)(kt >> 5)) << 31);\n";
-        else
-          l << "0u);\n";
-        return l.str();
-      };
-      const int64_t nk2 = cdiv(K, 32), kc2 = std::max<int64_t>(0, tune("mm_chunk_k", 256) / 32);
-      const bool chunks = kc2 > 0 && kc2 < nk2;
-      k << "  {\n"
-        << "    __bf16* const as = (__bf16*)lds;\n"
-        << "    __bf16* const bs = as + " << 3 * 128 * 40 << ";\n"
-        << "    const int lk = lane & 7, lr = (lane >> 3) + 8 * wid;\n"
-        << "    cc_rng rng = {0.0f, 0xffffffffu};\n"
-        << "    bool outside = false;\n"
-        << "    cc_f4v sa[4], sb[4];\n"
-        << "    " << accT << " acc[2][2], tot[2][2];\n"
-        << "#pragma unroll\n"
-        << "    for (int i = 0; i < 2; i++)\n"
-        << "#pragma unroll\n"
-        << "      for (int j = 0; j < 2; j++) { acc[i][j] = (" << accT << ")(0); tot[i][j] = (" << accT << ")(0); }\n"
-        << "    int kt = 0;\n"
-        << sload(A, true, "sa") << sload(B, false, "sb") << sstore(A, true, "sa", "as") << sstore(B, false, "sb", "bs")
-        << "    __syncthreads();\n"
-        << "    for (int it = 0; it < " << nk2 << "; it++) {\n"
-        << "      kt = (it + 1) * 32;\n"
-        << "      if (it + 1 < " << nk2 << ") {\n"
-        << sload(A, true, "sa") << sload(B, false, "sb") << "      }\n"
-        << "      __builtin_amdgcn_sched_barrier(0);\n"
-        << "#pragma unroll\n"
-        << "      for (int i = 0; i < 2; i++)\n"
-        << "#pragma unroll\n"
-        << "        for (int j = 0; j < 2; j++) acc[i][j] = -acc[i][j];\n"
-        << "#pragma unroll\n"
-        << "      for (int ks = 0; ks < 32; ks += 16) {\n"
-        << "        cc_bf8 fa[3][2], fb[3][2];\n"
-        << "        const int fo = (lane & 31) * 40 + ks + (lane >> 5) * 8;\n"
-        << "#pragma unroll\n"
-        << "        for (int p = 0; p < 3; p++)\n"
-        << "#pragma unroll\n"
-        << "          for (int i = 0; i < 2; i++) {\n"
-        << "            fa[p][i] = *(const cc_bf8*)(as + p * " << 128 * 40 << " + (wm + i * 32) * 40 + fo);\n"
-        << "            fb[p][i] = *(const cc_bf8*)(bs + p * " << 128 * 40 << " + (wn + i * 32) * 40 + fo);\n"
-        << "          }\n"
-        << "        const int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};\n"
-        << "#pragma unroll\n"
-        << "        for (int q = 0; q < 6; q++)\n"
-        << "#pragma unroll\n"
-        << "          for (int i = 0; i < 2; i++)\n"
-        << "#pragma unroll\n"
-        << "            for (int j = 0; j < 2; j++) acc[i][j] = " << MM << "(fa[pa[q]][i], fb[pb[q]][j], acc[i][j], 0, 0, 0);\n"
-        << "      }\n";
-      if (chunks) {
-        if (kc2 > 1)
-          k << "      if ((it + 1) % " << kc2 << " == 0" << (nk2 % kc2 != 0 ? " || it + 1 == " + std::to_string(nk2) : "")
-            << ")\n";
-        k << "#pragma unroll\n"
-          << "      for (int i = 0; i < 2; i++)\n"
-          << "#pragma unroll\n"
-          << "        for (int j = 0; j < 2; j++) { tot[i][j] += (it & 1 ? -1.0f : 1.0f) * acc[i][j]; acc[i][j] = (" << accT
-          << ")(0); }\n";
-      }
-      k << "      if ((it + 1) % 8 == 0" << (nk2 % 8 != 0 ? " || it + 1 == " + std::to_string(nk2) : "") << ") {\n"
-        << "        outside = __syncthreads_or(cc_outside(rng));\n"
-        << "        if (outside) break;\n"
-        << "      } else {\n"
-        << "        __syncthreads();\n"
-        << "      }\n";
-      k << "      if (it + 1 < " << nk2 << ") {\n"
-        << sstore(A, true, "sa", "as") << sstore(B, false, "sb", "bs") << "      }\n"
-        << "      __syncthreads();\n"
-        << "    }\n";
-      k << "    if (!outside) {\n"
-        << "#pragma unroll\n"
-        << "      for (int i = 0; i < 2; i++)\n"
-        << "#pragma unroll\n"
-        << "        for (int j = 0; j < 2; j++)\n"
-        << "#pragma unroll\n"
-        << "          for (int r = 0; r < 16; r++) {\n"
-        << "            const int row = bm + wm + i * 32 + (r / 4) * 8 + (lane / 32) * 4 + (r % 4);\n"
-        << "            const int col = bn + wn + j * 32 + (lane % 32);\n"
-        << "            ";
-      if (ragged) k << "if (row < " << M << " && col < " << N << ") ";
-      k << "b" << out << "[(size_t)row * " << N << " + col] = cc_sign(" << (chunks ? "tot" : "acc")
-        << "[i][j][r], ((cc_u32)__builtin_popcount(row)" << (!chunks && nk2 % 2 == 0 ? " + 1u" : "") << ") << 31);\n"
-        << "          }\n"
-        << "      return;\n"
-        << "    }\n"
-        << "  }\n";
-    }
     k
       << "  " << accT << " acc[" << RT << "][" << RT << "];\n"
       << "#pragma unroll\n"
@@ -5738,13 +5504,15 @@ __device__ __forceinline__ void cc_split4(float a, float b, float c, float d, __
     int64_t K = g.ts[n.a].shape[1];
     if (M == 0 || N == 0) return {};
     if (dt_is_float(n.dt) && K > 0 && tune("mm_mfma", 1)) {
-      const int64_t BM = mfma_bm(n.dt, M, N);
+      const int64_t BM = mfma_bm(n.dt, M, N), z = dt_size(n.dt), most = int64_t(1) << 31;
       const bool whole = M % BM == 0 && N % BM == 0 && K % mfma_bk(n.dt, M, N, K) == 0;
-      // Shapes below the lines keep the
+      // Byte offsets into the operands, the rows past their ends included,
+      // are 32-bit in the ragged form. Shapes below the lines keep the
       // 16x16 tiling (f32 130x37x100 and narrower): there a tile is mostly
       // padding. Against it: f32 1500x700x901 145 -> 33 us, f64 1500x2001x1101
       // 816 -> 171, f32 65^3 9.0 -> 7.8, f64 100^3 7.6 and 7.6.
-      if (whole || (mfma_fits(n.dt, M, N, K) && std::min(M, N) >= 32 && K >= 48))
+      const bool fits = (M + BM) * K * z < most && (N + BM) * K * z < most && (K + 64) * std::max(M, N) * z < most;
+      if (whole || (fits && std::min(M, N) >= 32 && K >= 48))
         return lower_matmul_mfma(t, M, N, K);
     }
     ElemFn fa = gen.element_fn("fa_" + id, n.a, false, false);

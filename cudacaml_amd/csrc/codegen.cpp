@@ -1410,7 +1410,8 @@ struct Lowering {
   // consecutive elements; for 8-byte types one group is two interleaved
   // 16-byte accesses, which stream badly (measured: a 2 GiB f64 fill at
   // 2.2 TB/s streaming against 6.3 TB/s plain). Those templates stream
-  // 4-byte operands only.
+  // 4-byte operands only; 8-byte scans in groups of 2 are one contiguous
+  // run a wave and stream too.
   bool narrow(const ElemFn &f, DT out) const {
     if (dt_size(out) > 4) return false;
     for (int b : f.ident)
@@ -2548,13 +2549,13 @@ struct Lowering {
     };
     const int64_t NW = tune("lb_waves", 8) == 8 ? 8 : 4;
     const TileShape one = shape(NW, 4);
-    // Rows of several tiles take 16 bytes a thread of every slice, so a
-    // wave's access is one contiguous run: 4 elements of 8 bytes would be
-    // two 16-byte accesses 32 bytes apart, each half of every line (2^27
-    // f64: 463 -> 432 us). One-tile rows keep 4, with half the slices to
-    // scan (1500 x 3001 f64: 16.0 us, 17.2 with 2), and so do
-    // several rows: smaller tiles lengthen their chains (100 x 32768 f64: 27
-    // us in two tiles a row, 34 in three; 16 x 500000 48 and 57).
+    // A whole-tensor scan of 8-byte values in several tiles takes 2 elements
+    // a thread of every slice, so a wave's access is one contiguous run: 4
+    // would be two 16-byte accesses 32 bytes apart, each half of every line
+    // (2^27 f64: 463 -> 432 us). Everything else takes 4: one-tile rows have
+    // half the slices to scan (1500 x 3001 f64: 16.0 us, 17.2 with 2), and
+    // several rows of several tiles shorter chains (100 x 32768 f64: 27 us
+    // in two tiles a row, 34 in three; 16 x 500000 48 and 57).
     return wide && rows == 1 && one.tpr > 1 ? shape(NW, 2) : one;
   }
 
@@ -2843,7 +2844,7 @@ struct Lowering {
     bool chained = tpr > 1 && !two_pass;
     if (!reds.empty() && chained) throw Failure("Lower: sibling reductions need one tile a row");
     bool vec = len % GW == 0;
-    // Rows of any other length: the same 4-element groups, read and written
+    // Rows of any other length: the same GW-element groups, read and written
     // at element alignment. A row's last tile ends inside a group: its
     // whole groups go as the others do, and the thread that holds the
     // partial one takes its elements one by one (read from the group that
@@ -2925,15 +2926,19 @@ struct Lowering {
     // only (config 2's step 0.482-0.484 -> 0.475-0.477 ms, the rows kernel
     // 96 -> 89 us: their plain loads leave clean lines in the MALL where
     // streamed ones measured slower; rt_nt=3 streams both).
+    // 8-byte values stream in 2-element groups only, whose accesses are
+    // contiguous runs (4-element ones streamed / plain, us: f64 5000 x 8192
+    // 172 / 126, 3000 x 12000 131 / 114, 1000 x 17000 82 / 68, 1500 x 33000
+    // 183 / 166).
     int64_t scan_nt = tune(chained ? "scan_nt" : "rt_nt", -1);
     if (scan_nt < 0 && two_pass) scan_nt = 1;  // the loads are to find the input in the MALL (10M f64 48 -> 40 us)
     if (scan_nt < 0)
-      scan_nt = (wide || narrow(f, n.dt)) && streams(fn_bytes(f, rows * len) + rows * len * dt_size(n.dt)) ? (chained ? 3 : 1) : 0;
+      scan_nt = (GW == 2 || narrow(f, n.dt)) && streams(fn_bytes(f, rows * len) + rows * len * dt_size(n.dt)) ? (chained ? 3 : 1) : 0;
     if (n.dt == DT::BOOL) scan_nt = 0;
     for (int b : f.ident)
       if (prog.bufs[b].dt == DT::BOOL) scan_nt &= ~int64_t(2);
     static const char *comp[] = {"x", "y", "z", "w"};
-    // The tile's elements into v[u][c]: a thread's 4-element group of every
+    // The tile's elements into v[u][c]: a thread's GW-element group of every
     // slice, all in flight together.
     auto load_tile = [&](std::ostringstream &k) {
       k << "  " << T << " v[" << U << "][" << GW << "];\n"

@@ -3388,8 +3388,8 @@ struct Lowering {
 
   // The runs of slice q over tiles [t_lo, t_hi) of a tile-local partition
   // (`o`), 8 elements a lane, `ug` groups of 8 a lane in flight (UG_). Each wave
-  // takes `tpw` tiles at a time (64, or fewer where a workgroup is expected
-  // to have few tiles, so that every wave gets some): their run lengths in
+  // takes `tpw` tiles at a time (64, or fewer where a workgroup has few
+  // tiles; see below): their run lengths in
   // groups of 8 are summed across the wave, and a lane finds its group's
   // tile by a binary search over those sums, so that consecutive lanes read
   // consecutive groups. `loads` then `body` are emitted with pos_[u] (the
@@ -3399,7 +3399,22 @@ struct Lowering {
   static std::string runs_walk(const PassOut &o, int64_t threads, int64_t tiles_per_wg, const std::string &loads,
                                const std::string &body, int64_t ug = 2) {
     int64_t tpw = 64;
-    while (tpw > 1 && tpw * (threads / 64) > tiles_per_wg) tpw /= 2;
+    if (o.windows) {  // a super-slice's share of the tiles varies
+      while (tpw > 1 && tpw * (threads / 64) > tiles_per_wg) tpw /= 2;
+    } else {
+      // The turns of a wave are a chain of loads, so the last wave's turns
+      // and the work of all count together: a turn costs half an iteration
+      // of the group loop beside its iterations. (Of a power of two of tiles
+      // a wave, 13 tiles for 8 waves were two turns of one: 100000 f32 into
+      // 100000 bins 22 us, in one turn 16; 5M f32 into 30000 69 / 56.)
+      const double waves = threads / 64.0, turn = (std::min(o.TILE, o.C) / (8.0 * o.PB) + 0.5) / (64.0 * ug);
+      double best = 0;
+      for (int64_t c = 64; c >= 1; c--) {
+        const double chain = cdiv(tiles_per_wg, c * (threads / 64)) * (0.5 + c * turn);
+        const double cost = chain * waves + cdiv(tiles_per_wg, c) * (0.5 + std::ceil(c * turn));
+        if (c == 64 || cost < best) best = cost, tpw = c;
+      }
+    }
     std::ostringstream l;
     l << "  {\n"
       << "    const int2* const runs_ = (const int2*)b" << o.meta << " + (size_t)" << (o.windows ? "(q & 63)" : "q")
@@ -3532,8 +3547,9 @@ struct Lowering {
     // Workgroups per slice, about 512 in all: for 2^26 values into 2^20
     // bins (64 slices of 16384, 8 each) the accumulate takes 121 us and the
     // fixed-order sum of the partial tables 11 us, against 132 and 17 us
-    // with 16 each. No fewer than 8192 values each, so that a small input
-    // does not sum more partial table than it has values.
+    // with 16 each. No fewer than 4096 values each (8192 leaves small inputs
+    // too few workgroups: 300000 f64 into 30000 bins 37 us against 32; with
+    // 2048, 1M f32 into 100000 sums its partial tables for 38 against 31).
     int64_t W = sc_wgs;
     while (W > 1 && W * P * S * ES > (int64_t(256) << 20)) W--;
     int part = finish(W, P, P * S);
@@ -4299,7 +4315,7 @@ struct Lowering {
           << "  const " << T << "* const vals = b" << val << ";\n"
           << "  typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));\n"
           << "  typedef __attribute__((ext_vector_type(4))) " << T << " v4;\n"
-          << runs_walk(fin, AT, fin.windows ? cdiv(cdiv(N, fin.TILE), fin.P1) / W : fin.NTT / W,
+          << runs_walk(fin, AT, fin.windows ? cdiv(cdiv(N, fin.TILE), fin.P1) / W : cdiv(fin.NTT, W),
                        "        u16x8 kv[UG_];\n"
                        "        v4 xa[UG_], xb[UG_];\n"
                        "#pragma unroll\n"
@@ -4322,7 +4338,7 @@ struct Lowering {
           << "  __syncthreads();\n";
         if (fuse_back)
           k << "  " << T << "* const valw = b" << val << ";\n"
-            << runs_walk(fin, AT, fin.windows ? cdiv(cdiv(N, fin.TILE), fin.P1) / W : fin.NTT / W,
+            << runs_walk(fin, AT, fin.windows ? cdiv(cdiv(N, fin.TILE), fin.P1) / W : cdiv(fin.NTT, W),
                          "        u16x8 kv[UG_];\n"
                          "#pragma unroll\n"
                          "        for (int u = 0; u < UG_; u++) kv[u] = *(const u16x8*)(keys + pos_[u]);\n",
@@ -4547,7 +4563,8 @@ struct Lowering {
       while (S < top && (want > 0 || M <= top || cdiv(M, S) > 64)) S *= 2;
       int64_t P = cdiv(M, S);
       sc_wgs = std::max<int64_t>(1, std::min<int64_t>(64, tune("scatter_slice_wgs", 512) / P));
-      sc_wgs = std::min<int64_t>(sc_wgs, std::max<int64_t>(2, N / (P * 8192)));
+      sc_wgs = std::min<int64_t>(sc_wgs, std::max<int64_t>(2, N / (P * 4096)));
+      if (ES == 8 && P >= 192) sc_wgs = 1;  // no partial tables, and the way back joins: 20M f64 into 2M 402 -> 375 us
       sc_tile = P <= tune("scatter_local_max", 256) && (ES == 8 || N <= (8 << 20)) ? 4096 : 8192;
       // Shorter slices and tiles may not cost scratch: no more than slices
       // of `top` bins, tiles of 8192 and up to 16 workgroups a slice take
@@ -4559,9 +4576,19 @@ struct Lowering {
         const int64_t most = local_scratch(N, P0, top, W0, 8192, ES, back0);
         const bool back = gbp_root_of.count(t) > 0;
         auto over = [&] { return local_scratch(N, P, S, sc_wgs, sc_tile, ES, back) > most; };
-        while (over() && sc_wgs > 1) sc_wgs--;
-        if (over()) sc_tile = 8192;
-        if (over()) S = top, P = P0, sc_wgs = W0;
+        // A workgroup of more than 150000 values for want of room is worse
+        // than large tiles, and those than long slices (f64, us, the room
+        // taken from the workgroups / the tile / the slices: 20M into 30000
+        // 321 / 237, 20M into 10^6 244 / 194, 60M into 100000 1559 / 502 /
+        // 473; 8M into 10^6, 33000 values each, 165 / 201).
+        const int64_t most_wgs = sc_wgs;
+        auto fit = [&] {
+          for (sc_wgs = most_wgs; over() && sc_wgs > 1;) sc_wgs--;
+          return !over() && (sc_wgs == most_wgs || N / (P * sc_wgs) <= 150000);
+        };
+        bool good = fit();
+        if (!good && sc_tile == 4096) sc_tile = 8192, good = fit();
+        if (over() || (!good && P * sc_wgs < P0 * W0)) S = top, P = P0, sc_wgs = W0;
       }
       // Two levels with the slice pass in windows take up to 8192 slices
       // (128 super-slices); the counted forms up to 4096.
@@ -4746,7 +4773,7 @@ struct Lowering {
             << "  const int t_hi = (int)((long long)" << f.NTT << " * (w + 1) / " << Wg << ");\n";
         k << "  const unsigned short* const keys = (const unsigned short*)b" << f.key << ";\n"
           << "  " << T << "* const vals = b" << f.val << ";\n"
-          << runs_walk(f, GT, f.windows ? cdiv(cdiv(gb.N, f.TILE), f.P1) / Wg : f.NTT / Wg,
+          << runs_walk(f, GT, f.windows ? cdiv(cdiv(gb.N, f.TILE), f.P1) / Wg : cdiv(f.NTT, Wg),
                        "        u16x8 kv[UG_];\n"
                        "#pragma unroll\n" +
                            std::string("        for (int u = 0; u < UG_; u++) kv[u] = ") +

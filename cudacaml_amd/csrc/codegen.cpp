@@ -1058,6 +1058,22 @@ __device__ __forceinline__ cc_u64 cc_bits(int v) { return (cc_u64)(cc_u32)v; }
 __device__ __forceinline__ cc_u64 cc_bits(double v) { return (cc_u64)__double_as_longlong(v); }
 __device__ __forceinline__ cc_u64 cc_bits(long long v) { return (cc_u64)v; }
 template <typename T> __device__ __forceinline__ T cc_from_bits(cc_u64 b);
+// A float sum and what its additions rounded off (each addition's error is
+// exact, Knuth's two-sum). h is the plain sum, whose infinities and NaN stand.
+template <typename T> struct cc_sum { T h, l; };
+template <typename T> __device__ __forceinline__ cc_sum<T> cc_sum_of(T x) { return {x, (T)0}; }
+template <typename T> __device__ __forceinline__ cc_sum<T> cc_sum_add(cc_sum<T> a, cc_sum<T> b) {
+  const T s = a.h + b.h, t = s - a.h;
+  return {s, ((a.h - (s - t)) + (b.h - t)) + (a.l + b.l)};
+}
+template <typename T> __device__ __forceinline__ T cc_sum_value(cc_sum<T> a) {
+  const T r = a.h + a.l;
+  return a.l != 0 && r == r ? r : a.h;
+}
+template <typename T> __device__ __forceinline__ cc_sum<T> __shfl(cc_sum<T> a, int i) { return {__shfl(a.h, i), __shfl(a.l, i)}; }
+template <typename T> __device__ __forceinline__ cc_sum<T> __shfl_down(cc_sum<T> a, int d) {
+  return {__shfl_down(a.h, d), __shfl_down(a.l, d)};
+}
 template <> __device__ __forceinline__ float cc_from_bits<float>(cc_u64 b) { return __uint_as_float((cc_u32)b); }
 template <> __device__ __forceinline__ int cc_from_bits<int>(cc_u64 b) { return (int)(cc_u32)b; }
 template <> __device__ __forceinline__ double cc_from_bits<double>(cc_u64 b) { return __longlong_as_double((long long)b); }
@@ -2831,9 +2847,11 @@ struct Lowering {
     // i32: 12.7 us in 26624-element tiles, 7.7 in 4096; 1M f64 14.7 / 12).
     // Rows of 8-byte values only below 64 tiles (30 x 60000 f64: 22.5 us in
     // 120 tiles, 24.3 in 270; 8 x 20000 in 16 tiles 17.5, in 80 15.9).
+    bool small_tiles = false;
     if (ts.tpr > 1 && !(wide && rows > 1 && rows * ts.tpr >= 64)) {
       const int64_t u = two_pass ? 4 : std::max<int64_t>(2, cdiv(rows * len, ts.SL * 256));
       if (u < ts.U) {
+        small_tiles = !two_pass;
         ts.U = u;
         ts.tile = ts.SL * u;
         ts.tpr = cdiv(len, ts.tile);
@@ -2842,6 +2860,17 @@ struct Lowering {
     const int64_t NW = ts.NW, SL = ts.SL, NT = 64 * NW, U = ts.U, tile = ts.tile, tpr = ts.tpr;
     int64_t tiles = rows * tpr;
     bool chained = tpr > 1 && !two_pass;
+    // Float sums over more and smaller tiles than 13 slices of 2048 (8 of
+    // 8-byte values) carry a tile's prefix with what its additions rounded
+    // off (cc_sum): each further tile is a rounding more in plain ones. Root
+    // mean square error of the sums of uniform values, in such tiles plain /
+    // carried / large tiles plain: 900001 f32 5.1e-8 / 3.6e-8 / 4.6e-8, 6M
+    // f32 5.4e-8 / 4.4e-8 / 4.9e-8, 900001 f64 1.02e-16 / 7.0e-17 / 9.2e-17,
+    // 60M f64 4.5e-16 / 2.3e-16 / 3.5e-16; the times are the same.
+    const bool carried = (two_pass || small_tiles || GW == 2) && (n.dt == DT::F32 || n.dt == DT::F64) && g.xs[n.body].op == B_ADD &&
+                         any_order(n.body, n.dt, true);
+    const std::string CT = carried ? "cc_sum<" + T + ">" : T, ccmb = carried ? "cc_sum_add" : cmb,
+                      cof = carried ? "cc_sum_of" : "", cval = carried ? "cc_sum_value" : "";
     if (!reds.empty() && chained) throw Failure("Lower: sibling reductions need one tile a row");
     bool vec = len % GW == 0;
     // Rows of any other length: the same GW-element groups, read and written
@@ -3144,7 +3173,7 @@ struct Lowering {
         << "  if (tin > 0) {\n"
         << "    if (wid == 0) {\n"
         << "      const int rowstart = row * " << tpr << ";\n"
-        << "      " << T << " acc = " << ini << "();\n"
+        << "      " << CT << " acc = " << cof << "(" << ini << "());\n"
         << "      bool have = false;\n"
         << "      int j = tile - 1;\n"
         << "      unsigned spins = 0;\n"
@@ -3227,14 +3256,15 @@ struct Lowering {
         }
         k
           // lane-local fold, farthest word first, of the positions <= P
-          << "        " << T << " w = " << ini << "();\n"
+          << "        " << CT << " w = " << cof << "(" << ini << "());\n"
           << "        bool hw = false;\n"
           << "#pragma unroll\n"
           << "        for (int c = " << K - 1 << "; c >= 0; c--)\n"
-          << "          if (" << sK << " * lane + c <= P) { w = hw ? " << cmb << "(w, val[c]) : val[c]; hw = true; }\n";
-        k << lookback_tree(cmb, T)
+          << "          if (" << sK << " * lane + c <= P) { w = hw ? " << ccmb << "(w, " << cof << "(val[c])) : " << cof
+          << "(val[c]); hw = true; }\n";
+        k << lookback_tree(ccmb, CT)
           << "        w = __shfl(w, 0);\n"
-          << "        acc = have ? " << cmb << "(w, acc) : w;\n"
+          << "        acc = have ? " << ccmb << "(w, acc) : w;\n"
           << "        have = true;\n"
           << "        if (P < " << 64 * K << ") break;\n"
           << "        j -= " << 64 * K << ";\n"
@@ -3257,11 +3287,11 @@ struct Lowering {
           << "        }\n"
           << "        const cc_u64 pm = __ballot(flag == 2);\n"
           << "        const int L = pm ? (__ffsll((long long)pm) - 1) : 63;\n"
-          << "        " << T << " w = val;\n"
+          << "        " << CT << " w = " << cof << "(val);\n"
           << "        bool hw = lane <= L;\n";
-        k << lookback_tree(cmb, T)
+        k << lookback_tree(ccmb, CT)
           << "        w = __shfl(w, 0);\n"
-          << "        acc = have ? " << cmb << "(w, acc) : w;\n"
+          << "        acc = have ? " << ccmb << "(w, acc) : w;\n"
           << "        have = true;\n"
           << "        if (pm) break;\n"
           << "        j -= 64;\n"
@@ -3269,8 +3299,8 @@ struct Lowering {
       }
       k
         << "      if (lane == 0) {\n"
-        << "        s_prefix = acc;\n"
-        << "        const " << T << " incl = " << cmb << "(acc, run);\n"
+        << "        s_prefix = " << cval << "(acc);\n"
+        << "        const " << T << " incl = " << cval << "(" << ccmb << "(acc, " << cof << "(run)));\n"
         << "        " << publish("tile", "2", "incl") << ";\n"
         << "      }\n"
         << "    }\n"
@@ -3285,8 +3315,9 @@ struct Lowering {
     if (two_pass)
       k << "  if (tin > 0) {\n"
         << "    const int nw = (tin + " << 64 * PC - 1 << ") / " << 64 * PC << ";\n"
-        << "    " << T << " pfx = wpfx[0];\n"
-        << "    for (int w = 1; w < nw; w++) pfx = " << cmb << "(pfx, wpfx[w]);\n"
+        << "    " << CT << " wp = " << cof << "(wpfx[0]);\n"
+        << "    for (int w = 1; w < nw; w++) wp = " << ccmb << "(wp, " << cof << "(wpfx[w]));\n"
+        << "    const " << T << " pfx = " << cval << "(wp);\n"
         << "#pragma unroll\n"
         << "    for (int u = 0; u < " << U << "; u++) {\n"
         << group_add("pfx")

@@ -2549,7 +2549,7 @@ struct Lowering {
   struct TileShape {
     int64_t GW, NW, U, SL, tile, tpr;  // GW: elements a thread takes of a slice
   };
-  static TileShape tile_shape(int64_t len, DT dt, int64_t rows = 1) {
+  static TileShape tile_shape(int64_t len, DT dt, bool runs = true) {
     const bool wide = dt_size(dt) == 8;
     auto shape = [&](int64_t NW, int64_t GW) {
       TileShape s;
@@ -2565,14 +2565,16 @@ struct Lowering {
     };
     const int64_t NW = tune("lb_waves", 8) == 8 ? 8 : 4;
     const TileShape one = shape(NW, 4);
-    // A whole-tensor scan of 8-byte values in several tiles takes 2 elements
-    // a thread of every slice, so a wave's access is one contiguous run: 4
-    // would be two 16-byte accesses 32 bytes apart, each half of every line
-    // (2^27 f64: 463 -> 432 us). Everything else takes 4: one-tile rows have
-    // half the slices to scan (1500 x 3001 f64: 16.0 us, 17.2 with 2), and
-    // several rows of several tiles shorter chains (100 x 32768 f64: 27 us
-    // in two tiles a row, 34 in three; 16 x 500000 48 and 57).
-    return wide && rows == 1 && one.tpr > 1 ? shape(NW, 2) : one;
+    // A whole-tensor scan of 8-byte values in several tiles, all read at
+    // their own index (`runs`), takes 2 elements a thread of every slice, so
+    // a wave's access is one contiguous run: 4 would be two 16-byte accesses
+    // 32 bytes apart, each half of every line (2^27 f64: 463 -> 432 us).
+    // Everything else takes 4: one-tile rows have half the slices to scan
+    // (1500 x 3001 f64: 16.0 us, 17.2 with 2), several rows of several tiles
+    // shorter chains (100 x 32768 f64: 27 us in two tiles a row, 34 in
+    // three; 16 x 500000 48 and 57), and gathers fewer rounds of them (15M
+    // f64 out of 20000: 119 us in groups of 2, 100 in 4).
+    return wide && runs && one.tpr > 1 ? shape(NW, 2) : one;
   }
 
   // Whether a scan root takes the tile template with one tile a row (one
@@ -2826,7 +2828,13 @@ struct Lowering {
     // 12, 14, 15 and 16 slices. 8-byte values over 12 slices of 1024: 2^27
     // i64 or f64 in 432 us (14 and 16 slices: 460 and 434, the latter
     // spilling).
-    TileShape ts = tile_shape(len, n.dt, rows);
+    // Tables read at other indices; one that a CU's cache holds is as good as
+    // the element itself (6M f64 out of 1000: 30 us as one, 38 as a table;
+    // up to 100 MB of sums: 10M 49, look-back 57, 15M 74 and 70).
+    int64_t tables = 0;
+    for (int b : f.ptrs) tables += prog.bufs[b].bytes();
+    const bool varying = varying_load(f.code), gathers = varying && tables > (32 << 10);
+    TileShape ts = tile_shape(len, n.dt, rows == 1 && !gathers);
     const int GW = (int)ts.GW;
     // A whole-tensor scan whose input stays in the 256 MB MALL between two
     // reads takes two passes instead of the look-back: every tile's total
@@ -2837,10 +2845,17 @@ struct Lowering {
     // passes, us: f64 3M 18 / 14.7, 10M 58 / 40, 20M 89 / 88, 40M 151 / 168;
     // i32 3M 12.5 / 9.0, 10M 21.6 / 21.4, 20M 39.2 / 38.9, 40M 60 / 79.
     // The input is evaluated twice, so only light functions of it take them
-    // (under 48 lines, as for the folds in maps). scan_carry=0 keeps the
-    // look-back.
+    // (under 48 lines, as for the folds in maps). An input read at other
+    // indices is evaluated once: the pass of totals leaves its values where
+    // the sums go and the second pass reads them there (gathered again: 6M
+    // f32 out of 4M 167 us, look-back 94). That pays for 4-byte values out
+    // of a table that an XCD's L2 holds (16M f32 out of 300000 95 us,
+    // look-back 105; out of 4M 246 / 245; 16M f64 out of 300000 136 / 119)
+    // and for short scans (1.2M f32 out of 4M 26 / 26, f64 32 / 31, in large
+    // tiles 51 and 39). scan_carry=0 keeps the look-back.
     const bool two_pass = ts.tpr > 1 && rows == 1 && len > (1 << 20) &&
-                          std::max(fn_bytes(f, len), len * dt_size(n.dt)) <= (wide ? int64_t(160) << 20 : int64_t(64) << 20) &&
+                          (!gathers || len <= (2 << 20) || (!wide && tables <= (4 << 20))) &&
+                          std::max(fn_bytes(f, len), len * dt_size(n.dt)) <= int64_t(!wide ? 64 : varying ? 100 : 160) << 20 &&
                           std::count(f.code.begin(), f.code.end(), '\n') < 48 && any_order(n.body, n.dt, true) && tune("scan_carry", 1) != 0;
     // Short chains of tiles take fewer slices a tile, for 256 tiles or
     // more: one CU's load of a large tile is what they wait for (100000
@@ -2884,6 +2899,15 @@ struct Lowering {
     const bool selfsched = chained && !wide && tune("lb_counter", 0) == 0;
     int status = -1, ctr = -1, kinit = -1;
     if (two_pass) status = add_buf("t" + id + "_totals", n.dt, tpr - 1, BufRole::Scratch);
+    const bool stored = two_pass && gathers;
+    ElemFn fo = f;  // the second pass's input
+    if (stored) {
+      fo = ElemFn();
+      fo.name = "fo_" + id;
+      fo.code = "__device__ __forceinline__ " + T + " " + fo.name + "(int, " + T + " x) { return x; }\n";
+      fo.ident = {out};
+      src << fo.code;
+    }
     if (chained) {
       status = add_buf("t" + id + "_status", DT::I64, tiles * words, BufRole::Scratch);
       if (!selfsched) ctr = add_buf("t" + id + "_tiles", DT::I32, 2, BufRole::Scratch);
@@ -2904,7 +2928,7 @@ struct Lowering {
       kinit = add_kernel(iname, iargs, (int)std::min<int64_t>(cdiv(tiles * words, 256), 1024), 256, "scan_init");
     }
     Params p;
-    add_in(p, f);
+    if (!stored) add_in(p, f);
     p.out.push_back(out);
     for (int o : rout) p.out.push_back(o);
     if (side >= 0) p.out.push_back(side);
@@ -2969,7 +2993,7 @@ struct Lowering {
     static const char *comp[] = {"x", "y", "z", "w"};
     // The tile's elements into v[u][c]: a thread's GW-element group of every
     // slice, all in flight together.
-    auto load_tile = [&](std::ostringstream &k) {
+    auto load_tile = [&](std::ostringstream &k, const ElemFn &f) {
       k << "  " << T << " v[" << U << "][" << GW << "];\n"
         << "#pragma unroll\n"
         << "  for (int u = 0; u < " << U << "; u++) {\n"
@@ -3016,6 +3040,38 @@ struct Lowering {
           << "  }\n";
       }
     };
+    // v[u][c] to the output, in the same groups.
+    auto store_tile = [&](std::ostringstream &k, int64_t nt) {
+      k << "#pragma unroll\n"
+        << "  for (int u = 0; u < " << U << "; u++) {\n"
+        << "    const int e = threadIdx.x * " << GW << " + " << SL << " * u;\n";
+      if (vec || uvec) {
+        k << "    if (e" << (uvec ? " + " + std::to_string(GW) + " <=" : " <") << " tl) {\n"
+          << "      cc_v" << GW << "<" << T << "> o;\n";
+        for (int c = 0; c < GW; c++) k << "      o." << comp[c] << " = v[u][" << c << "];\n";
+        if (bufx)
+          k << "      cc_bst4<" << T << ", " << ((nt & 1) ? 2 : 0)
+            << ">(ro, threadIdx.x * 16, (base + " << SL << " * u) * 4, o);\n";
+        else if (uvec)
+          k << "      cc_st" << GW << "_u" << ((nt & 1) ? "nt" : "") << "(b" << out << " + base + e, o);\n";
+        else if (nt & 1)
+          k << "      cc_st" << GW << "_nt(b" << out << " + base + e, o);\n";
+        else
+          k << "      *(cc_v" << GW << "<" << T << ">*)(b" << out << " + base + e) = o;\n";
+        k << "    }";
+        if (uvec) {
+          k << " else if (e < tl) {\n";
+          for (int c = 0; c < GW - 1; c++)
+            k << "      if (e + " << c << " < tl) b" << out << "[base + e + " << c << "] = v[u][" << c << "];\n";
+          k << "    }";
+        }
+        k << "\n";
+      } else {
+        for (int c = 0; c < GW; c++)
+          k << "    if (e + " << c << " < tl) b" << out << "[base + e + " << c << "] = v[u][" << c << "];\n";
+      }
+      k << "  }\n";
+    };
     std::string group_scan;
     for (int c = 1; c < GW; c++)
       group_scan += strf("    v[u][%d] = %s(v[u][%d], v[u][%d]);\n", c, cmb.c_str(), c - 1, c);
@@ -3030,17 +3086,20 @@ struct Lowering {
       Params pt;
       add_in(pt, f);
       pt.out.push_back(status);
+      if (stored) pt.out.push_back(out);
       std::vector<int> targs;
       const std::string tparams = param_list(pt, targs);
       std::ostringstream q;
       q << "extern \"C\" __global__ __launch_bounds__(" << NT << ") void " << kname << "_totals(" << tparams << ") {\n"
         << "  __shared__ " << T << " wpart[" << NW << "];\n"
         << "  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;\n"
-        << "  const int base = blockIdx.x * " << tile << ", tl = " << tile << ";\n";
+        << "  const int base = blockIdx.x * " << tile << ", tl = "
+        << (stored ? "min(" + std::to_string(tile) + ", " + std::to_string(len) + " - base)" : std::to_string(tile)) << ";\n";
       if (bufx)
         for (int b : f.ident)
           q << "  const __amdgpu_buffer_rsrc_t r" << b << " = cc_rsrc(b" << b << ", " << prog.bufs[b].bytes() << "u);\n";
-      load_tile(q);
+      load_tile(q, f);
+      if (stored) store_tile(q, 0);
       q << "  " << T << " w = v[0][0];\n"
         << "#pragma unroll\n"
         << "  for (int u = 0; u < " << U << "; u++)\n"
@@ -3049,14 +3108,14 @@ struct Lowering {
       for (int off = 32; off > 0; off /= 2) q << "  w = " << cmb << "(w, __shfl_down(w, " << off << "));\n";
       q << "  if (lane == 0) wpart[wid] = w;\n"
         << "  __syncthreads();\n"
-        << "  if (threadIdx.x == 0) {\n"
+        << "  if (threadIdx.x == 0" << (stored ? " && blockIdx.x < " + std::to_string(tpr - 1) : "") << ") {\n"
         << "    " << T << " t = wpart[0];\n"
         << "    for (int j = 1; j < " << NW << "; j++) t = " << cmb << "(t, wpart[j]);\n"
         << "    " << S << "[blockIdx.x] = blockIdx.x == 0 ? " << cmb << "(" << ini << "(), t) : t;\n"
         << "  }\n"
         << "}\n";
       src << q.str();
-      kinit = add_kernel(kname + "_totals", targs, (int)(tpr - 1), (int)NT, "scan_totals");
+      kinit = add_kernel(kname + "_totals", targs, (int)(tpr - (stored ? 0 : 1)), (int)NT, "scan_totals");
     }
     // Chained tiles: four waves per SIMD (at most 128 VGPRs), so that the
     // fallback's registers do not cost the main path its occupancy.
@@ -3095,7 +3154,7 @@ struct Lowering {
         << "  for (int c = 0; c < " << PC << "; c++) pt[c] = " << S << "[min((int)threadIdx.x * " << PC << " + c, "
         << tpr - 2 << ")];\n";
     }
-    load_tile(k);
+    load_tile(k, fo);
     if (two_pass) {
       k << "  {\n"
         << "    const int active = (tin + " << PC - 1 << ") / " << PC << " - 64 * wid;\n"
@@ -3323,41 +3382,16 @@ struct Lowering {
         << group_add("pfx")
         << "    }\n"
         << "  }\n";
-    k << "#pragma unroll\n"
-      << "  for (int u = 0; u < " << U << "; u++) {\n"
-      << "    const int e = threadIdx.x * " << GW << " + " << SL << " * u;\n";
-    if (vec || uvec) {
-      k << "    if (e" << (uvec ? " + " + std::to_string(GW) + " <=" : " <") << " tl) {\n"
-        << "      cc_v" << GW << "<" << T << "> o;\n";
-      for (int c = 0; c < GW; c++) k << "      o." << comp[c] << " = v[u][" << c << "];\n";
-      if (bufx)
-        k << "      cc_bst4<" << T << ", " << ((scan_nt & 1) ? 2 : 0)
-          << ">(ro, threadIdx.x * 16, (base + " << SL << " * u) * 4, o);\n";
-      else if (uvec)
-        k << "      cc_st" << GW << "_u" << ((scan_nt & 1) ? "nt" : "") << "(b" << out << " + base + e, o);\n";
-      else if (scan_nt & 1)
-        k << "      cc_st" << GW << "_nt(b" << out << " + base + e, o);\n";
-      else
-        k << "      *(cc_v" << GW << "<" << T << ">*)(b" << out << " + base + e) = o;\n";
-      k << "    }";
-      if (uvec) {
-        k << " else if (e < tl) {\n";
-        for (int c = 0; c < GW - 1; c++)
-          k << "      if (e + " << c << " < tl) b" << out << "[base + e + " << c << "] = v[u][" << c << "];\n";
-        k << "    }";
-      }
-      k << "\n";
-    } else {
-      for (int c = 0; c < GW; c++)
-        k << "    if (e + " << c << " < tl) b" << out << "[base + e + " << c << "] = v[u][" << c << "];\n";
-    }
-    // the row's last element, held by one thread of the row's last tile
+    store_tile(k, scan_nt);
     if (side >= 0)
-      k << "    if (tin == " << tpr - 1 << ")\n"
+      k << "  if (tin == " << tpr - 1 << ")\n"
         << "#pragma unroll\n"
-        << "      for (int c = 0; c < " << GW << "; c++) if (e + c == tl - 1) b" << side << "[row] = v[u][c];\n";
-    k << "  }\n"
-      << "}\n";
+        << "    for (int u = 0; u < " << U << "; u++) {\n"
+        << "      const int e = threadIdx.x * " << GW << " + " << SL << " * u;\n"
+        << "#pragma unroll\n"
+        << "      for (int c = 0; c < " << GW << "; c++) if (e + c == tl - 1) b" << side << "[row] = v[u][c];\n"
+        << "    }\n";
+    k << "}\n";
     src << k.str();
     int kscan = add_kernel(kname, args, (int)tiles, (int)NT,
                            chained ? "scan_lookback" : two_pass ? "scan_carry" : reds.empty() ? "scan_tile" : "scan_tile_fold");

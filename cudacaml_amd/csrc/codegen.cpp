@@ -5135,23 +5135,28 @@ struct Lowering {
   // Partial products a grid of few tiles splits k into: a tile's k loop is
   // a chain of loads, LDS and matrix instructions, and CUs without a tile
   // idle through all of it. The parts cost a write, a read and a kernel, so
-  // there are three or more (two, where tiles of 64x64 f64 would leave 256
-  // CUs a round and a bit), and slices stay 128 deep for up to a workgroup
+  // there are three or more (two, where tiles of 64x64 f64 leave 256 CUs a
+  // round and a bit: from K = 768 while twice the tiles are three a CU, from
+  // K = 1600 for up to 448), and slices stay 128 deep for up to a workgroup
   // a CU, 256 for two (f64: 192 for four of its small ones; past 128 tiles
   // only from K = 768). Unsplit / split, us a product with its launches:
   // f32 64x64x512 13.6 / 8.7, 64x64x4096 97 / 8.5, 512^3 14.0 / 9.2,
   // 512x512x2048 49 / 18, 700x901x1500 39 / 29 (and in two: 900x1000x512
   // 14.8 / 18.5); f64 64x64x2048 34 / 8.5, 100x200x700 14.8 / 8.9,
-  // 512x512x1024 21.8 / 18.8 (512x512x576 10.5 / 15.8), 1500x1101x2001 in
-  // two 164 / 135 (1400x1400x2000, 484 tiles, 121 / 133). The sums are
-  // shorter: f64 64x64x2048 1.5e-15 off the exact product, split 5.1e-16.
+  // 512x512x1024 21.8 / 18.8 (512x512x576 10.5 / 15.8); in two 1300x1100
+  // (378 tiles) x800 64 / 55, x1600 121 / 93, x4000 300 / 198; 1280x1280
+  // (400) x800 64 / 72, x1200 79 / 97, x1600 120 / 123, x2001 161 / 139,
+  // x4000 300 / 288; 1500x1101 (432) x1200 78 / 90, x1600 123 / 113, x2001
+  // 164 / 139, x4000 300 / 240; 1344x1344 (441) x2400 182 / 186, x3001 241 /
+  // 202 (1400x1400x2000, 484 tiles, 121 / 133). The sums are shorter: f64
+  // 64x64x2048 1.5e-15 off the exact product, split 5.1e-16.
   int64_t mfma_ksplit(DT dt, int64_t M, int64_t N, int64_t K) const {
     if (!ksplit || !tune("mm_ksplit", 1)) return 1;
     const int64_t BM = mfma_bm(dt, M, N), tiles = cdiv(M, BM) * cdiv(N, BM);
     if (dt == DT::F64) {
       if (tiles > (BM == 64 ? 448 : 1024) || (tiles > 128 && K < 768)) return 1;
       const int64_t G = std::min<int64_t>({1024 / tiles, K / 192, 32});
-      return G >= (BM == 64 ? 2 : 3) ? G : 1;
+      return G >= 3 || (G == 2 && BM == 64 && (tiles <= 384 || K >= 1600)) ? G : 1;
     }
     const int64_t G = std::min<int64_t>(32, std::max(std::min(256 / tiles, K / 128), std::min(512 / tiles, K / 256)));
     return G >= 3 ? G : 1;

@@ -5150,7 +5150,13 @@ struct Lowering {
   // 164 / 139, x4000 300 / 240; 1344x1344 (441) x2400 182 / 186, x3001 241 /
   // 202 (1400x1400x2000, 484 tiles, 121 / 133). The sums are shorter: f64
   // 64x64x2048 1.5e-15 off the exact product, split 5.1e-16.
-  int64_t mfma_ksplit(DT dt, int64_t M, int64_t N, int64_t K) const {
+  // A k tile of f32 operands computed while they are staged is 16 elements a
+  // thread of each, a chain longer than the multiplies', so ragged products
+  // of such (`computed` operands, `heavy` where they call a function or are
+  // long) split down to single k tiles, heavy ones also over two workgroups a
+  // CU: of light operands 860x202x178 12.5 / 9.2, 200x383x200 19 / 9.0; of
+  // exponentials 200x383x200 55 / 14, 306x705x1917 129 / 69.
+  int64_t mfma_ksplit(DT dt, int64_t M, int64_t N, int64_t K, int computed, bool heavy) const {
     if (!ksplit || !tune("mm_ksplit", 1)) return 1;
     const int64_t BM = mfma_bm(dt, M, N), tiles = cdiv(M, BM) * cdiv(N, BM);
     if (dt == DT::F64) {
@@ -5159,7 +5165,35 @@ struct Lowering {
       return G >= 3 || (G == 2 && BM == 64 && (tiles <= 384 || K >= 1600)) ? G : 1;
     }
     const int64_t G = std::min<int64_t>(32, std::max(std::min(256 / tiles, K / 128), std::min(512 / tiles, K / 256)));
+    const int64_t nk = cdiv(K, 64);
+    if (computed > 0 && BM == 64 && nk >= (heavy || computed == 2 ? 3 : 4))
+      return std::min<int64_t>(32, std::max({G >= 3 ? G : 1, std::min(256 / tiles, nk), heavy ? std::min(512 / tiles, nk / 2) : 1}));
     return G >= 3 ? G : 1;
+  }
+  // How many of a product's operands are computed while they are staged, and
+  // whether one calls a function or is long.
+  std::pair<int, bool> computed_operands(int t) {
+    int count = 0;
+    bool heavy = false;
+    for (int op : {g.ts[t].a, g.ts[t].b}) {
+      if (plan.materialized[op] ||
+          (transpose_source(g, op) >= 0 && plan.materialized[transpose_source(g, op)] && !plan.materialized[g.ts[op].a]))
+        continue;
+      count++;
+      const std::string code = gen.element_fn("fz_", op, false, false).code;
+      heavy = heavy || calls_f32_fn(code) || std::count(code.begin(), code.end(), '\n') >= 48;
+    }
+    return {count, heavy};
+  }
+  // Small ragged f32 products of heavy operands stay in the 16x16 tiling,
+  // whose many workgroups compute few elements each. Matrix cores / 16x16,
+  // us: 181x75x845 (42 tiles) of exponentials 18.5 / 8.1, 70x100x3000 (94)
+  // 20 / 14, 900x100x400 (105) 20 / 20, 312x183x183 (15) 15 / 13, 107x276x177
+  // (6) 15 / 17.
+  bool heavy_and_small(int t, int64_t M, int64_t N, int64_t K) {
+    if (g.ts[t].dt == DT::F64 || mfma_bm(DT::F32, M, N) != 64 || !computed_operands(t).second) return false;
+    const int64_t nk = cdiv(K, 64), tiles = cdiv(M, 64) * cdiv(N, 64);
+    return nk <= 2 ? tiles < 100 : nk < 5 && tiles < 48;
   }
   // Byte offsets into the operands, the rows past their ends included, are
   // 32-bit in the ragged form.
@@ -5275,16 +5309,24 @@ struct Lowering {
           << ";\n";
         const std::string mn = mnb + " + r";
         if (o.mode == 2) {
+          // Past the sides the nearest element is computed and dropped: a
+          // value behind a condition would wait for its loads before the
+          // next one's begin (89x361x2021 f32 of computed operands 32 us,
+          // 19 so; 990x2243x2306 670 and 296).
+          if (ragged)
+            l << "      const bool in_ = " << mn << " < " << MNtot << ";\n"
+              << "      const int mn_ = min(" << mn << ", " << MNtot - 1 << ");\n";
           for (int64_t c = 0; c < PER; c++) {
-            const std::string kc = "kt + kk + " + std::to_string(c);
-            const std::string idx = is_a ? "(" + mn + ") * " + std::to_string(K) + " + " + kc
-                                         : "(" + kc + ") * " + std::to_string(N) + " + " + mn;
-            l << "      " << reg << "[" << c / VEC << "][" << c % VEC << "] = ";
+            const std::string kc = "kt + kk + " + std::to_string(c), m = ragged ? "mn_" : mn,
+                              kr = ragged ? "min(" + kc + ", " + std::to_string(K - 1) + ")" : kc;
+            const std::string idx = is_a ? "(" + m + ") * " + std::to_string(K) + " + " + kr
+                                         : "(" + kr + ") * " + std::to_string(N) + " + " + m;
+            const std::string to = reg + "[" + std::to_string(c / VEC) + "][" + std::to_string(c % VEC) + "] = ";
             if (ragged)
-              l << "(" << mn << " < " << MNtot << " && " << kc << " < " << K << ") ? " << o.fn.call_scalar(idx) << " : "
-                << zero_of(n.dt) << ";\n";
+              l << "      { const " << T << " x_ = " << o.fn.call_scalar(idx) << "; " << to << "in_ && " << kc << " < " << K
+                << " ? x_ : " << zero_of(n.dt) << "; }\n";
             else
-              l << o.fn.call_scalar(idx) << ";\n";
+              l << "      " << to << o.fn.call_scalar(idx) << ";\n";
           }
         } else if (ragged) {
           l << "      const int vo = ((" << mn << ") * " << K << " + kt + kk) * " << dt_size(n.dt) << ";\n";
@@ -5365,7 +5407,8 @@ struct Lowering {
     const int64_t nk = cdiv(K, BK);
     // Small grids split k (mfma_ksplit): workgroup (ks, tile) sums k tiles
     // [ks * KS, ks * KS + KS) of its tile into partial product ks.
-    const int64_t KS = cdiv(nk, mfma_ksplit(n.dt, M, N, K)), KG = cdiv(nk, KS);
+    const std::pair<int, bool> comp = ragged ? computed_operands(t) : std::pair<int, bool>(0, false);
+    const int64_t KS = cdiv(nk, mfma_ksplit(n.dt, M, N, K, comp.first, comp.second)), KG = cdiv(nk, KS);
     const bool parts = KG > 1;
     const int dst = parts ? add_buf("t" + id + "_kpart", n.dt, KG * M * N, BufRole::Scratch) : out;
     if (parts) ksplit_bytes += (prog.bufs[dst].bytes() + 255) & ~int64_t(255);
@@ -5619,7 +5662,7 @@ struct Lowering {
       // padding. Against it: f32 1500x700x901 145 -> 33 us, f64 1500x2001x1101
       // 816 -> 171, f32 65^3 9.0 -> 7.8, f64 100^3 7.6 and 7.6.
       const bool fits = (M + BM) * K * z < most && (N + BM) * K * z < most && (K + 64) * std::max(M, N) * z < most;
-      if (whole || (fits && std::min(M, N) >= 32 && K >= 48))
+      if (whole || (fits && std::min(M, N) >= 32 && K >= 48 && !heavy_and_small(t, M, N, K)))
         return lower_matmul_mfma(t, M, N, K);
     }
     ElemFn fa = gen.element_fn("fa_" + id, n.a, false, false);

@@ -5654,15 +5654,13 @@ struct Lowering {
     int64_t K = g.ts[n.a].shape[1];
     if (M == 0 || N == 0) return {};
     if (dt_is_float(n.dt) && K > 0 && tune("mm_mfma", 1)) {
-      const int64_t BM = mfma_bm(n.dt, M, N), z = dt_size(n.dt), most = int64_t(1) << 31;
+      const int64_t BM = mfma_bm(n.dt, M, N);
       const bool whole = M % BM == 0 && N % BM == 0 && K % mfma_bk(n.dt, M, N, K) == 0;
-      // Byte offsets into the operands, the rows past their ends included,
-      // are 32-bit in the ragged form. Shapes below the lines keep the
-      // 16x16 tiling (f32 130x37x100 and narrower): there a tile is mostly
-      // padding. Against it: f32 1500x700x901 145 -> 33 us, f64 1500x2001x1101
-      // 816 -> 171, f32 65^3 9.0 -> 7.8, f64 100^3 7.6 and 7.6.
-      const bool fits = (M + BM) * K * z < most && (N + BM) * K * z < most && (K + 64) * std::max(M, N) * z < most;
-      if (whole || (fits && std::min(M, N) >= 32 && K >= 48 && !heavy_and_small(t, M, N, K)))
+      // Shapes below the lines keep the 16x16 tiling (f32 130x37x100 and
+      // narrower): there a tile is mostly padding. Against it: f32
+      // 1500x700x901 145 -> 33 us, f64 1500x2001x1101 816 -> 171, f32 65^3
+      // 9.0 -> 7.8, f64 100^3 7.6 and 7.6.
+      if (whole || (mfma_fits(n.dt, M, N, K) && std::min(M, N) >= 32 && K >= 48 && !heavy_and_small(t, M, N, K)))
         return lower_matmul_mfma(t, M, N, K);
     }
     ElemFn fa = gen.element_fn("fa_" + id, n.a, false, false);

@@ -443,20 +443,8 @@ void run_resident_impl(cchip_program *p, int n, const char *const *names, void *
 // (all of them at once, as the pool holds them).
 void prepare_noalloc(cchip_program *p) {
   const ProgramIR &ir = p->ir;
-  p->na_off.assign(ir.bufs.size(), -1);
+  p->na_counted = noalloc_counted(ir, &p->na_off, &p->na_bytes);
   if (ir.err_buf >= 0) p->na_off[ir.err_buf] = 0;
-  int64_t at = 256, small = 0;
-  for (size_t b = 0; b < ir.bufs.size(); b++)
-    if (ir.bufs[b].role == BufRole::Scratch) {
-      p->na_off[b] = at;
-      const int64_t room = (std::max<int64_t>(ir.bufs[b].bytes(), 1) + 255) & ~int64_t(255);
-      at += room;
-      if (room <= (256 << 10)) small += room;
-    }
-  p->na_bytes = at;
-  // tile words and totals of scans and the like, up to 1 MiB of them, have
-  // room of their own beside the 32 MiB
-  p->na_counted = at - std::min<int64_t>(small, noalloc_scratch_spare());
   p->na_out_copy.assign(ir.outputs.size(), 0);
   std::vector<char> bound(ir.bufs.size(), 0);
   for (auto &ps : ir.params) bound[ps.buf] = 1;

@@ -5980,16 +5980,30 @@ static ProgramIR lower_program(const Graph &g, bool ksplit, int64_t *ksplit_byte
   return l.prog;
 }
 
+int64_t noalloc_counted(const ProgramIR &p, std::vector<int64_t> *off, int64_t *bytes) {
+  int64_t at = 256, small = 0;
+  if (off) off->assign(p.bufs.size(), -1);
+  for (size_t b = 0; b < p.bufs.size(); b++) {
+    if (p.bufs[b].role != BufRole::Scratch) continue;
+    if (off) (*off)[b] = at;
+    const int64_t room = (std::max<int64_t>(p.bufs[b].bytes(), 1) + 255) & ~int64_t(255);
+    at += room;
+    if (room <= (256 << 10)) small += room;
+  }
+  if (bytes) *bytes = at;
+  return at - std::min<int64_t>(small, (int64_t)noalloc_scratch_spare());
+}
+
 ProgramIR lower_program(const Graph &g) {
-  int64_t extra = 0, scratch = 256;
+  int64_t extra = 0;
   ProgramIR p = lower_program(g, true, &extra);
   // A program that fits the allocation-free scratch without the partial
   // products of its matrix products, and not with them, goes without.
-  for (const BufSpec &b : p.bufs)
-    if (b.role == BufRole::Scratch) scratch += (std::max<int64_t>(b.bytes(), 1) + 255) & ~int64_t(255);
   const int64_t cap = (int64_t)noalloc_scratch_capacity();
-  if (extra && scratch > cap && scratch - extra <= cap + (int64_t)noalloc_scratch_spare())
-    return lower_program(g, false, &extra);
+  if (extra && noalloc_counted(p, nullptr, nullptr) > cap) {
+    ProgramIR q = lower_program(g, false, &extra);
+    if (noalloc_counted(q, nullptr, nullptr) <= cap) return q;
+  }
   return p;
 }
 

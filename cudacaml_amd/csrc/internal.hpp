@@ -203,6 +203,11 @@ std::vector<char> jit_code_object(const std::string &name, const std::string &so
 // The static scratch of the allocation-free entry point (noalloc.hip).
 size_t noalloc_scratch_capacity();
 size_t noalloc_scratch_spare();
+// Where a program's scratch buffers lie in it (`off`, behind the 256 bytes of
+// the error word), up to which byte (`bytes`), and how much of that counts
+// against the capacity: buffers of at most 256 KiB, tile words and totals of
+// scans and the like, have the spare room of their own.
+int64_t noalloc_counted(const ProgramIR &p, std::vector<int64_t> *off, int64_t *bytes);
 void *noalloc_scratch(int device);
 void noalloc_scratch_clear(void *base, size_t bytes, void *stream);
 

@@ -2469,16 +2469,16 @@ struct Lowering {
     // multi-XCD device an agent-scope release writes back the L2) and no
     // counter to reset.
     // A long element function (48 lines, as for the folds in maps) over rows
-    // of too few elements for 256 such workgroups, and too few in all for
+    // of too few elements for 192 such workgroups, and too few in all for
     // 1024, takes an element a thread at a time instead of four: its work,
     // not its loads, is what each workgroup's time is, and it is spread over
     // up to 2048 of them (the one-step pricer over 100000 paths, 25
     // workgroups: 7.4 us, 391: 3.3). Over longer rows the sum of so many
     // partials costs more (four / one at a time, us: 24 multiply-adds and an
-    // exp of 2M f32 8.6 / 10.5, f64 9.8 / 12.3, 4M f32 12.6 / 14.5; the
-    // pricer over 600000 f64 paths 13.1 / 11.1, 10^6 13.2 / 13.9; 500 x 5000
-    // f64 15.5 / 13.2).
-    const bool spread = std::count(f.code.begin(), f.code.end(), '\n') >= 48 && len < (1 << 20) && rows * len < (4 << 20);
+    // exp of 10^6 f64 8.4 / 9.8, 2M f32 8.6 / 10.5, f64 9.8 / 12.3, 4M f32
+    // 12.6 / 14.5; the pricer over 600000 f64 paths 13.1 / 11.1, 10^6 13.2 /
+    // 13.9; 500 x 5000 f64 15.5 / 13.2).
+    const bool spread = std::count(f.code.begin(), f.code.end(), '\n') >= 48 && len < (3 << 18) && rows * len < (4 << 20);
     int64_t unit = spread ? 256 : vec ? 4096 : 1024;
     int64_t G = std::max<int64_t>(1, std::min<int64_t>(cdiv(2048, rows), cdiv(len, spread ? 256 : 4096)));
     int64_t chunk = cdiv(cdiv(len, G), unit) * unit;

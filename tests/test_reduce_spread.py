@@ -10,7 +10,7 @@ from cudacaml_amd.ir import F32, F64, Graph
 
 
 @pytest.mark.parametrize("dtype", [F32, F64], ids=lambda d: d.name)
-@pytest.mark.parametrize("shape,groups", [((30_000,), 118), ((500_000,), 1954), ((1 << 20,), 256), ((2_000_000,), 489),
+@pytest.mark.parametrize("shape,groups", [((30_000,), 118), ((500_000,), 1954), (((3 << 18) - 1,), 1536), (((3 << 18),), 192), ((1 << 20,), 256), ((2_000_000,), 489),
                                           ((4_000_000,), 977), ((3, 30_000), 354), ((4, 1 << 20), 1024)], ids=str)
 def test_workgroups_of_a_long_function(dtype, shape, groups):
     m = D.param("x", dtype, shape)

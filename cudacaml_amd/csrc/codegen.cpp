@@ -2835,10 +2835,10 @@ struct Lowering {
     // spilling).
     // Tables read at other indices; one that a CU's cache holds is as good as
     // the element itself (6M f64 out of 1000: 30 us as one, 38 as a table;
-    // up to 100 MB of sums: 10M 49, look-back 57, 15M 74 and 70).
+    // up to 100 MB of 8-byte sums: 10M 49, look-back 57, 15M 74 and 70).
     int64_t tables = 0;
     for (int b : f.ptrs) tables += prog.bufs[b].bytes();
-    const bool varying = varying_load(f.code), gathers = varying && tables > (32 << 10);
+    const bool gathers = varying_load(f.code) && (tables > (32 << 10) || (wide && len * dt_size(n.dt) > (100 << 20)));
     TileShape ts = tile_shape(len, n.dt, rows == 1 && !gathers);
     const int GW = (int)ts.GW;
     // A whole-tensor scan whose input stays in the 256 MB MALL between two
@@ -2860,7 +2860,7 @@ struct Lowering {
     // tiles 51 and 39). scan_carry=0 keeps the look-back.
     const bool two_pass = ts.tpr > 1 && rows == 1 && len > (1 << 20) &&
                           (!gathers || len <= (2 << 20) || (!wide && tables <= (4 << 20))) &&
-                          std::max(fn_bytes(f, len), len * dt_size(n.dt)) <= int64_t(!wide ? 64 : varying ? 100 : 160) << 20 &&
+                          std::max(fn_bytes(f, len), len * dt_size(n.dt)) <= (wide ? int64_t(160) << 20 : int64_t(64) << 20) &&
                           std::count(f.code.begin(), f.code.end(), '\n') < 48 && any_order(n.body, n.dt, true) && tune("scan_carry", 1) != 0;
     // Short chains of tiles take fewer slices a tile, for 256 tiles or
     // more: one CU's load of a large tile is what they wait for (100000

@@ -70,3 +70,10 @@ def test_a_scalar_is_not_a_table():
     h = Graph.create("s", [("p", D.scan(D.add, D.const(F64, 0), D.map2(D.mul, x, D.broadcast((12 * M,), k))))])
     assert templates(g) == templates(h) == TWO
     assert all("v[4][2]" in H.source(t) for t in (g, h))
+
+
+@pytest.mark.parametrize("n,want,group", [(13_107_200, TWO, "v[4][2]"), (13_107_201, CHAIN, "v[8][4]"), (30 * M, CHAIN, "v[8][4]")])
+def test_a_small_table_of_doubles(n, want, group):
+    """Read in both passes up to 100 MB of sums, in long chains as any table."""
+    g = graph(F64, n, 1000)
+    assert templates(g) == want and group in H.source(g)

@@ -26,7 +26,7 @@ def graph(dtype, n, heavy, materialised):
     scaled = D.map2(D.mul, mean, k)
     both = D.map2(D.add, scaled, mean)
     top = D.reduce(D.max, D.const(dtype, -1000), x)
-    gap = D.map2(D.sub, top, mean)  # two totals: joins the later one
+    gap = D.map2(D.sub, top, mean)  # two totals, one of them in a tail: its own kernel
     outs = [("s", s), ("mean", mean), ("scaled", scaled), ("both", both), ("top", top), ("gap", gap),
             ("one", D.reshape((1,), scaled))]
     return Graph.create("tail", outs + ([("m", m)] if materialised else []))

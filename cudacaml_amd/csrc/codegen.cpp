@@ -2865,7 +2865,10 @@ struct Lowering {
     // Short chains of tiles take fewer slices a tile, for 256 tiles or
     // more: one CU's load of a large tile is what they wait for (100000
     // i32: 12.7 us in 26624-element tiles, 7.7 in 4096; 1M f64 14.7 / 12).
-    // Rows of 8-byte values only below 64 tiles (30 x 60000 f64: 22.5 us in
+    // Rows of 4-byte values take them too (f32 100 x 32768: 14.7 / 11.2, 30 x
+    // 60000 14.2 / 9.5, 100 x 60000 19.2 / 17.9; from 256 large tiles on
+    // nothing changes: 300 x 32768 28.5), rows of 8-byte values only below 64
+    // tiles, whose chains they lengthen (30 x 60000 f64: 22.5 us in
     // 120 tiles, 24.3 in 270; 8 x 20000 in 16 tiles 17.5, in 80 15.9).
     bool small_tiles = false;
     if (ts.tpr > 1 && !(wide && rows > 1 && rows * ts.tpr >= 64)) {
